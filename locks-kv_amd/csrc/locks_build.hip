@@ -11,18 +11,18 @@
 //   ms = max(|mu| / 127, 1e-8); muq = clamp(rint(mu / ms), +-127)
 //   scales stored bf16 (RNE); tag = K[15, kh, 0:8].
 //
-// MI355X mapping: one wave per (block, kv head).  The page is staged in LDS
-// as fp32; the gram runs on v_mfma_f32_16x16x4_f32 (A and B operands are the
-// same lane values because Gm = dc dc^T); the eigendecomposition is a
-// parallel cyclic Jacobi (round-robin ordering: 8 disjoint rotations per
-// step, 15 steps per sweep) on the 16x16 matrix in LDS -- the reference
-// calls a batched LAPACK/cuSOLVER eigh; any eigensolver agrees with it only
-// up to eigenvector sign/rotation, which the summary tolerates by design.
-// The quantize/pack stage is shared with locks_pack_rki4, which takes the
-// eigenpairs from the caller and is bit-exact to the reference op order
-// (V accumulated over t in ascending order with separately rounded multiply
-// and add, IEEE division, round-half-even).
+// MI355X mapping: a wave builds 64 / page pages at once, a page on `page`
+// lanes, with the gram and the eigenvectors in registers (rki4_build_kernel).
+// The gram runs on v_mfma_f32_16x16x4_f32 (A and B operands are the same lane
+// values because Gm = dc dc^T); the eigendecomposition is a parallel cyclic
+// Jacobi (round-robin ordering: page / 2 disjoint rotations per step, page - 1
+// steps per sweep) -- the reference calls a batched LAPACK/cuSOLVER eigh; any
+// eigensolver agrees with it only up to eigenvector sign/rotation, which the
+// summary tolerates by design.  locks_pack_rki4 takes the eigenpairs from the
+// caller and follows the reference's op order (V accumulated over t in
+// ascending order, IEEE division, round-half-even), which the build shares.
 #include <algorithm>
+#include <type_traits>
 
 #include "locks_common.h"
 #include "locks_hip.h"
@@ -32,30 +32,20 @@ namespace locks {
 constexpr int BD_RNK = 8;
 // build grid cap (waves stride over the rest): a few resident rounds on 256 CUs
 constexpr long BD_MAX_GRID = 4096;
+// items up to which a wave builds one page instead of 64 / page: one wave per
+// SIMD of the chip (1024 pages: 60 us one a wave; 1600 to 4096: 70 us at four)
+constexpr long BD_SPREAD = 1024;
 
-// Per-wave LDS image of one (block, kv head) page of PG tokens x D dims.
+// Per-wave LDS image of one page of locks_pack_rki4: PG tokens x D dims and
+// the caller's eigenvectors.
 template <int D, int PG>
 struct WaveLds {
     float dc[PG][D + 1];         // centred page (padded rows)
     float mu[D];
-    float A[PG][PG + 1];         // gram, rotated in place
-    float U[PG][PG + 1];         // accumulated eigenvectors (columns)
-    // second buffers of the page-64 Jacobi step (one element per row 1 x 1
-    // otherwise)
-    float A2[PG == 64 ? PG : 1][PG + 1];
-    float U2[PG == 64 ? PG : 1][PG + 1];
-    float cc[PG], ss[PG];
+    float U[PG][PG + 1];         // eigenvectors (columns)
     float S8[BD_RNK];
     int col[BD_RNK];             // eigen column of basis r (ascending top-8)
-    float red[BD_RNK][kWave / 8];
 };
-// waves per workgroup: as many page images as fit 160 KB of LDS, at most 4;
-// d = 512 (the MLA latent, ~37 KB per image) runs one
-template <int D, int PG> constexpr int bd_waves() {
-    if (D >= 512) return 1;
-    constexpr int n = (160 * 1024) / (int)sizeof(WaveLds<D, PG>);
-    return n >= 4 ? 4 : n;
-}
 
 // quantize + pack one page from mu (LDS), dc (LDS), U8 = U[:, col[r]],
 // S8 (LDS), writing the six slab rows.  Lane l owns the packed bytes
@@ -74,12 +64,10 @@ __device__ __forceinline__ void pack_page(WaveLds<D, PG>& L, long row, const Sla
             const int d = 2 * (lane + 64 * k) + e;
 #pragma unroll
             for (int r = 0; r < BD_RNK; ++r) {
-                // d <= 256: a compiler barrier keeps one column's operands
-                // live at a time (hoisting all 16 x 8 basis values costs ~130
-                // VGPRs and halves the occupancy).  d = 512 runs one wave per
-                // SIMD anyway (its LDS image), so there the hoisting is free
-                // and the barrier would only multiply the LDS reloads.
-                if constexpr (D <= 256) asm volatile("" ::: "memory");
+                // a compiler barrier keeps one column's operands live at a
+                // time (hoisting all 16 x 8 basis values costs ~130 VGPRs and
+                // halves the occupancy)
+                asm volatile("" ::: "memory");
                 float acc = 0.f;
                 const int c = L.col[r];
                 if (own(k))
@@ -141,219 +129,470 @@ __device__ __forceinline__ void pack_page(WaveLds<D, PG>& L, long row, const Sla
     if (lane == 0) *reinterpret_cast<uint16_t*>(S.mus + row * S.smus) = f32_to_bf16(msc);
 }
 
-// Parallel cyclic Jacobi on L.A (N x N symmetric, N = page = 16, 32 or 64);
-// eigenvectors -> L.U columns.  Round-robin pairing of step `step`: index 0
-// stays, 1..N-1 rotate; the pair of position k (1 <= k < N/2) is
-// (at(k), at(N-1-k)), position 0 pairs index 0 with at(0), where
-// at(k) = 1 + (k + step) % (N - 1).
+__device__ __forceinline__ long readlane64(long v, int l) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)v, l), hi = (uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l);
+    return (long)(((uint64_t)hi << 32) | lo);
+}
+// value of another lane; addr = 4 x lane
+__device__ __forceinline__ float from_lane(int addr, float v) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
+}
+// a in the lanes of mask m, b in the others.  Selects are spelled by mask: as
+// conditionals on a lane's own index the compiler makes the row array an
+// indexed one, in scratch memory.
+__device__ __forceinline__ float pick(uint64_t m, float a, float b) {
+    return __builtin_amdgcn_inverse_ballot_w64(m) ? a : b;
+}
+// a in lane I of every page, b elsewhere.  The mask is made where it is used
+// (scalar moves): as plain constants the masks of all I are hoisted together
+// and spilled to VGPR lanes, a read each.
+template <int N, int I>
+__device__ __forceinline__ float pick_lane(float a, float b) {
+    constexpr uint64_t M = (N == 16 ? 0x0001000100010001ull : N == 32 ? 0x0000000100000001ull : 1ull) << I;
+    uint32_t lo, hi;
+    asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"((int)(uint32_t)M));
+    if constexpr ((uint32_t)(M >> 32) == (uint32_t)M) hi = lo;
+    else asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((int)(uint32_t)(M >> 32)));
+    return pick(((uint64_t)hi << 32) | lo, a, b);
+}
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
+// sum over the N lanes of a page, result in each
 template <int N>
-__device__ __forceinline__ int rr_at(int k, int step) { return 1 + (k + step) % (N - 1); }
-template <int N>
-__device__ __forceinline__ int rr_partner(int i, int step) {
-    if (i == 0) return rr_at<N>(0, step);
-    const int k = (i - 1 - step + (N - 1)) % (N - 1);
-    return k == 0 ? 0 : rr_at<N>(N - 1 - k, step);
+__device__ __forceinline__ float lanes_sum(float v) {
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    v += row_ror<1>(v);
+    if constexpr (N >= 32) v = xor16_sum(v);
+    if constexpr (N >= 64) v = xor32_sum(v);
+    return v;
 }
 
-// Parallel cyclic Jacobi on the N x N symmetric matrix in L.A (eigenvalues
-// end on the diagonal, eigenvectors in the columns of L.U).  One step applies
-// the N/2 disjoint rotations of the round-robin schedule as one two-sided
-// update A'' = J^T A J read entirely from the old A:
+// ---- build ------------------------------------------------------------------
+// One wave builds up to 64 / PG pages at once: a page of PG tokens is PG
+// lanes, and lane j holds column j of the page's gram and row j of its
+// eigenvectors in registers (2 PG VGPRs), so the row half of a Jacobi rotation
+// is register arithmetic and only the gram's column half moves data between
+// lanes (PG ds_bpermute per step, no LDS storage).  With one page per wave and
+// both matrices in LDS the build was bound by its LDS accesses (page 16: ~47
+// per step and page) and, one page alone, by their latency.  Same roundings in
+// the same order, so the records keep their bytes.  Measured, before -> after:
+//   8 layers x 2048 pages x 8 heads, d 128 page 16   4.06 -> 0.91 ms (7.0 ns a page)
+//   8 layers x 2048 latent pages, d 512              1.20 -> 0.26 ms
+//   4 layers x 512 pages x 8 heads, d 128 page 32    6.52 -> 0.96 ms
+//   4 layers x 256 pages x 8 heads, d 128 page 64    135 -> 3.85 ms
+//   32 layers x 8 heads x 4 pages (one a wave)       82 -> 60 us
+// Page 16 is now bound by VALU issue: 150 of a step's ~165 instructions are
+// VALU, four steps' worth of pages at once; the gram and the pack are 1/4.
+
+// Parallel cyclic Jacobi, round-robin ordering: index 0 stays, 1 .. N - 1
+// rotate.  At step s index i > 0 sits in slot 1 + (i - 1 - s) mod (N - 1);
+// slot 0 (index 0) pairs with slot 1, slot m > 1 with slot N + 1 - m; a pair is
+// (p, q) with p in slot 0 or 2 .. N / 2.  Rows are kept in slot order: a step
+// writes each row one slot down, so every step is the same code.  One step
+// applies the N / 2 disjoint rotations as A'' = J^T A J from the old A:
 //   A''[i][j] = c_j (c_i A[i][j] + s_i A[pi][j]) + s_j (c_i A[i][pj] + s_i A[pi][pj])
 //   U'[i][j]  = c_j U[i][j] + s_j U[i][pj]
-// Lane l owns column j = l % N of rows l / N + (64 / N) e.  A wave executes
-// its LDS instructions in order, so the old values every lane reads are read
-// before any lane writes (the asm barriers keep the compiler from moving the
-// accesses across each other): two dependent LDS round trips per step.
+// A is kept by columns (lane j: column j), U by rows (lane t: row t, its
+// columns in slot order too), so only A's column half needs an exchange.
 // Rotation parameters use the hardware reciprocal and reciprocal square root
 // (~1 ulp): a rotation only has to reduce the off-diagonal mass, and the
 // result is checked through the quantised summary, not bit for bit.
-template <int N, class W>
-__device__ void jacobi(W& L) {
+// `cs`: this page's N / 2 (c, s) pairs in LDS.  On return `diag` is the
+// eigenvalue of column j = lane % N and U the eigenvectors' entries of token j.
+template <int N>
+__device__ __forceinline__ void jacobi(float (&A)[N], float (&U)[N], float& diag, float2* cs, int lane) {
     static_assert(N == 16 || N == 32 || N == 64, "page 16, 32 or 64");
-    constexpr int RS = kWave / N, RPL = N * N / kWave;   // row stride, rows per lane
     constexpr int SWEEPS = N == 16 ? 12 : N == 32 ? 16 : 20;
-    const int lane = threadIdx.x & 63;
-    const int j = lane % N, r0 = lane / N;
-    for (int i = lane; i < N * N; i += kWave) L.U[i / N][i % N] = (i / N == i % N) ? 1.f : 0.f;
-    wave_lds_sync();
+    const int base = lane & ~(N - 1);
+    bool done = false;
+#pragma unroll 1
     for (int sweep = 0; sweep < SWEEPS; ++sweep) {
-        // convergence test: off-diagonal mass vs diagonal
-        float off = 0.f, dia = 0.f;
-        for (int i = lane; i < N * N; i += kWave) {
-            const float a = L.A[i / N][i % N];
-            if (i / N == i % N) dia += a * a; else off += a * a;
-        }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            off += __shfl_xor(off, o, kWave);
-            dia += __shfl_xor(dia, o, kWave);
-        }
-        // wave-uniform (also exits on 0/0).  fp32 rounding leaves off/dia
-        // near 1e-14 (asymmetric residues of order eps * |lambda|), so the
-        // bound sits above that floor: 5-6 sweeps at N = 16 instead of
-        // running out the sweep limit, with the same top-8 eigenvalue
-        // accuracy (~3e-6 rel).
-        if (!(off > 1e-12f * dia)) break;
+        // Off-diagonal mass against the diagonal, per page (also done on 0/0).
+        // fp32 rounding leaves off/dia near 1e-14 (asymmetric residues of
+        // order eps * |lambda|), so the bound sits above that floor: 5-6 sweeps
+        // at N = 16 instead of running out the sweep limit, with the same top-8
+        // eigenvalue accuracy (~3e-6 rel).
+        float off = 0.f, dia = diag * diag;
+        static_for<0, N>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const float a = pick_lane<N, i>(0.f, A[i]);
+            off = __builtin_fmaf(a, a, off);
+        });
+        off = lanes_sum<N>(off);
+        dia = lanes_sum<N>(dia);
+        done = done || !(off > 1e-12f * dia);
+        if (__ballot(!done) == 0) break;
+        int slot = lane & (N - 1);
+        // (three steps a turn where they divide the sweep: results then land
+        // in their registers without moves)
+#pragma unroll N == 32 ? 1 : 3
         for (int step = 0; step < N - 1; ++step) {
-            // page 64: A / U alternate between the two buffers step by step
-            float (*Ac)[N + 1] = (N == 64 && (step & 1)) ? L.A2 : L.A;
-            if (lane < N / 2) {
-                const int p = lane == 0 ? 0 : rr_at<N>(lane, step);
-                const int q = lane == 0 ? rr_at<N>(0, step) : rr_at<N>(N - 1 - lane, step);
-                const float apq = Ac[p][q], app = Ac[p][p], aqq = Ac[q][q];
-                float c = 1.f, sn = 0.f;
-                if (fabsf(apq) > 1e-30f) {                 // smaller: nothing to rotate away
-                    const float theta = (aqq - app) * __builtin_amdgcn_rcpf(2.f * apq);
-                    const float t = copysignf(__builtin_amdgcn_rcpf(fabsf(theta) +
-                                                                    __builtin_amdgcn_sqrtf(theta * theta + 1.f)),
-                                              theta);
-                    c = __builtin_amdgcn_rsqf(t * t + 1.f);
-                    sn = t * c;
-                }
-                L.cc[p] = c; L.ss[p] = -sn;
-                L.cc[q] = c; L.ss[q] = sn;
-            }
-            asm volatile("" ::: "memory");
-            const int pj = rr_partner<N>(j, step);
-            const float cj = L.cc[j], sj = L.ss[j];
-            if constexpr (N == 64) {
-                // 64 rows per lane: read the current buffers, write the
-                // other ones (the old values are never overwritten inside the
-                // step, so nothing has to be held in registers), then swap
-                float (*Uc)[N + 1] = (step & 1) ? L.U2 : L.U;
-                float (*An)[N + 1] = (step & 1) ? L.A : L.A2;
-                float (*Un)[N + 1] = (step & 1) ? L.U : L.U2;
-                for (int i = 0; i < N; ++i) {
-                    const int pi = rr_partner<N>(i, step);
-                    const float ci = L.cc[i], si = L.ss[i];
-                    An[i][j] = cj * (ci * Ac[i][j] + si * Ac[pi][j]) + sj * (ci * Ac[i][pj] + si * Ac[pi][pj]);
-                    Un[i][j] = cj * Uc[i][j] + sj * Uc[i][pj];
-                }
-                asm volatile("" ::: "memory");
-                continue;
-            }
-            float na[RPL], nu[RPL];
+            const int ps = slot < 2 ? 1 - slot : N + 1 - slot;       // the partner's slot and lane
+            int pi = ps + step;
+            pi = pi >= N ? pi - (N - 1) : pi;
+            pi = ps == 0 ? 0 : pi;
+            const int addr = (base | pi) << 2;
+            const float pd = from_lane(addr, diag);
+            // this column's element in the partner's row
+            float t[N / 2];
+            const uint64_t odd = __ballot(ps & 1);
 #pragma unroll
-            for (int e = 0; e < RPL; ++e) {
-                const int i = r0 + RS * e, pi = rr_partner<N>(i, step);
-                const float ci = L.cc[i], si = L.ss[i];
-                na[e] = cj * (ci * L.A[i][j] + si * L.A[pi][j]) + sj * (ci * L.A[i][pj] + si * L.A[pi][pj]);
-                nu[e] = cj * L.U[i][j] + sj * L.U[i][pj];
-            }
-            asm volatile("" ::: "memory");
+            for (int i = 0; i < N / 2; ++i) t[i] = pick(odd, A[2 * i + 1], A[2 * i]);
 #pragma unroll
-            for (int e = 0; e < RPL; ++e) {
-                L.A[r0 + RS * e][j] = na[e];
-                L.U[r0 + RS * e][j] = nu[e];
+            for (int b = 2, n = N / 4; n >= 1; b *= 2, n /= 2) {
+                const uint64_t m = __ballot(ps & b);
+#pragma unroll
+                for (int i = 0; i < n; ++i) t[i] = pick(m, t[2 * i + 1], t[2 * i]);
+            }
+            const float po = from_lane(addr, t[0]);
+            // first of its pair (p): slot 0 or 2 .. N / 2
+            const uint64_t first = __ballot(((slot == 0) | ((unsigned)(slot - 2) <= (unsigned)(N / 2 - 2))) != 0);
+            const float sgn = pick(first, 1.f, -1.f);
+            const float apq = pick(first, po, t[0]);                 // A[p][q] is column q's
+            // A[q][q] - A[p][p], the same on both lanes down to the zero's sign
+            const float theta = __builtin_fmaf(pd, sgn, -(diag * sgn)) * __builtin_amdgcn_rcpf(2.f * apq);
+            const float tt = copysignf(__builtin_amdgcn_rcpf(fabsf(theta) +
+                                                             __builtin_amdgcn_sqrtf(__builtin_fmaf(theta, theta, 1.f))),
+                                       theta);
+            const float cr = __builtin_amdgcn_rsqf(__builtin_fmaf(tt, tt, 1.f));
+            const bool rot = !done && fabsf(apq) > 1e-30f;           // smaller: nothing to rotate away
+            const float c = rot ? cr : 1.f, sn = rot ? tt * cr : 0.f;
+            const float sj = -sgn * sn;
+            const int e = min(slot, ps);                             // the pair's place: p's slot, 0 and 2 .. N / 2
+            cs[e == 0 ? 0 : e - 1] = make_float2(c, sn);             // (both lanes of the pair: the same value)
+            asm volatile("" ::: "memory");
+            // the diagonal element, with the roundings of the full update
+            const float d0 = __builtin_fmaf(c, diag, sj * t[0]), d1 = __builtin_fmaf(c, po, sj * pd);
+            const float nd = __builtin_fmaf(c, d0, sj * d1);
+            diag = done ? diag : nd;
+            float B[N], W[N];
+#pragma unroll
+            for (int k = 0; k < N / 2; ++k) {
+                const float2 r = cs[k];
+                const int p = k == 0 ? 0 : k + 1, q = k == 0 ? 1 : N - k;
+                B[p] = __builtin_fmaf(r.x, A[p], -(r.y * A[q]));
+                B[q] = __builtin_fmaf(r.x, A[q], r.y * A[p]);
+                W[p] = __builtin_fmaf(r.x, U[p], -(r.y * U[q]));
+                W[q] = __builtin_fmaf(r.x, U[q], r.y * U[p]);
             }
             asm volatile("" ::: "memory");
-        }
-        if constexpr (N == 64) {
-            // a sweep has 63 steps: the result sits in the second buffers
-            for (int i = 0; i < N; ++i) {
-                L.A[i][lane] = L.A2[i][lane];
-                L.U[i][lane] = L.U2[i][lane];
-            }
-            asm volatile("" ::: "memory");
+            // (issued together: left to the scheduler each exchange is waited
+            // for before the next goes out, 82 -> 72 us for 1024 single pages)
+            float pb[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) pb[i] = from_lane(addr, B[i]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                A[i == 0 ? 0 : i == 1 ? N - 1 : i - 1] = __builtin_fmaf(c, B[i], sj * pb[i]);
+#pragma unroll
+            for (int i = 0; i < N; ++i) U[i == 0 ? 0 : i == 1 ? N - 1 : i - 1] = W[i];
+            slot = slot < 2 ? (slot == 0 ? 0 : N - 1) : slot - 1;
         }
     }
 }
 
-// eigenvalues on the diagonal of L.A -> ascending ranks -> top-8 columns
-template <int N, class W>
-__device__ void select_top8(W& L) {
-    const int lane = threadIdx.x & 63;
-    if (lane < N) {
-        const float li = L.A[lane][lane];
-        int rank = 0;
-        for (int j = 0; j < N; ++j) {
-            const float lj = L.A[j][j];
-            rank += (lj < li) || (lj == li && j < lane);
-        }
-        if (rank >= N - BD_RNK) {
-            const int r = rank - (N - BD_RNK);
-            L.col[r] = lane;
-            L.S8[r] = __fsqrt_rn(fmaxf(li, 1e-10f));
-        }
-    }
-    wave_lds_sync();
+// a / b, correctly rounded, from y = RN(1 / b): the quotient estimate a y and
+// one residual correction (Markstein 1990; exact away from under- / overflow).
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
 }
 
-// Grid: capped, waves stride over (layer, block, kv head).  Layer l reads K from
-// k_layers[l] (or kc for a single-layer call) and writes slab rows offset by
-// l * layer_rows.  n_dev, when given, is a device count of valid entries of
-// `blocks` (at most n_blocks): the refresh producers size the grid to the
-// host-known bound and the list is compacted on the device.
-template <int D, int PG = 16>
-__global__ __launch_bounds__((bd_waves<D, PG>() * kWave)) void rki4_build_kernel(
+typedef const __attribute__((address_space(1))) uint32_t* global_u32;
+
+// Per-wave LDS: a window of one page's centred channels for the gram (pitch a
+// multiple of 4 words that is odd in quads, so the operand reads spread over
+// all banks), then the rotation pairs, then the kept columns of every page
+// with their singular values and reciprocals.
+template <int PG>
+struct BuildLds {
+    static constexpr int GW = kWave / PG;            // pages per wave
+    static constexpr int WIN = 128 * 16 / PG;        // channels per window
+    union {
+        float dc[PG][WIN + 4];
+        float2 cs[GW][PG / 2];
+        struct {
+            float u[GW][BD_RNK][PG];
+            float s8[GW][BD_RNK], y8[GW][BD_RNK];
+            uint32_t lam[kWave];
+        } top;
+    };
+};
+
+// Grid: one wave per gpw (1 to 64 / PG) consecutive (layer, block, kv head)
+// items, waves stride over the rest.  Layer l reads K from k_layers[l] (or kc
+// for a single-layer call) and writes slab rows offset by l * layer_rows.
+// n_dev, when given, is a device count of valid entries of `blocks` (at most
+// n_blocks): the refresh producers size the grid to the host-known bound and
+// the list is compacted on the device.
+template <int D, int PG>
+__global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_kernel(
     const uint16_t* __restrict__ kc, const uint64_t* __restrict__ k_layers,
     long k_sb, long k_st, long k_sh, int NB,
     const int* __restrict__ blocks, const int* __restrict__ n_dev, int n_blocks, int n_kv,
-    int n_layers, long layer_rows, SlabRows S, uint16_t* __restrict__ tag)
+    int n_layers, long layer_rows, SlabRows S, uint16_t* __restrict__ tag, int gpw)
 {
-    constexpr int NW = bd_waves<D, PG>();
-    __shared__ WaveLds<D, PG> lds[NW];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    WaveLds<D, PG>& L = lds[wave];
+    using LDS = BuildLds<PG>;
+    constexpr int NW = 4, GW = LDS::GW, NB16 = PG / 16;
+    constexpr int LPP = D >= 128 ? 64 : D / 2;       // lanes that share a page's channels
+    constexpr int NK = D >= 128 ? D / 128 : 1;       // 128-channel groups; lane l: channels 2 l, 2 l + 1 of each
+    constexpr int WIN = LDS::WIN, WCH = D < WIN ? D : WIN, NWIN = (D < 128 ? D : 128) / WCH;
+    __shared__ __attribute__((aligned(16))) LDS lds[NW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    LDS& L = lds[wave];
     const int nb_valid = n_dev ? min(*n_dev, n_blocks) : n_blocks;
-    const long per_layer = (long)nb_valid * n_kv;
-    // one wave per (layer, block index, kv head), grid-stride
-    for (long item = (long)blockIdx.x * NW + wave; item < per_layer * n_layers;
-         item += (long)gridDim.x * NW) {
-        const int layer = (int)(item / per_layer);
-        const long rem = item - (long)layer * per_layer;
-        const int bi = (int)(rem / n_kv), kh = (int)(rem % n_kv);
-        const int blk = blocks[bi];
-        if (blk < 0 || blk >= NB) continue;                        // masked (profile pass)
-        const long row = (long)layer * layer_rows + (long)blk * n_kv + kh;
-        const uint16_t* kbase = k_layers ? reinterpret_cast<const uint16_t*>(k_layers[layer]) : kc;
-        const uint16_t* kp = kbase + (long)blk * k_sb + (long)kh * k_sh;
-
-        // stage K (fp32) and the centroid (sequential sum over t, then / PG)
-        for (int i = lane; i < PG * D / 8; i += kWave) {
-            const int t = i / (D / 8), d0 = (i % (D / 8)) * 8;
-            const uint4 w = *reinterpret_cast<const uint4*>(kp + (long)t * k_st + d0);
-            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                L.dc[t][d0 + 2 * e] = bf16lo(ws[e]);
-                L.dc[t][d0 + 2 * e + 1] = bf16hi(ws[e]);
+    const long per_layer = (long)nb_valid * n_kv, total = per_layer * n_layers;
+    const int j = lane & (PG - 1), pg = lane / PG;   // this lane's column / token, and page
+    const bool own = lane < LPP;                     // d = 64: the upper lanes repeat, and store nothing
+    const int cl = own ? lane : lane - LPP;
+    for (long base = ((long)blockIdx.x * NW + wave) * gpw; base < total; base += (long)gridDim.x * NW * gpw) {
+        // this lane's page: K address (null: none) and summary row
+        const uint16_t* kpl = nullptr;
+        long rwl = 0;
+        if (pg < gpw && base + pg < total) {
+            const long it = base + pg;
+            const int layer = total <= 0xFFFFFFFFL ? (int)((uint32_t)it / (uint32_t)per_layer) : (int)(it / per_layer);
+            const uint32_t rem = (uint32_t)(it - (long)layer * per_layer);      // < n_blocks * n_kv
+            const uint32_t bi = rem / (uint32_t)n_kv;
+            const int blk = blocks[bi];
+            if (blk >= 0 && blk < NB) {                                // else masked (profile pass)
+                const int kh = (int)(rem - bi * (uint32_t)n_kv);
+                rwl = (long)layer * layer_rows + (long)blk * n_kv + kh;
+                kpl = (k_layers ? reinterpret_cast<const uint16_t*>(k_layers[layer]) : kc) +
+                      (long)blk * k_sb + (long)kh * k_sh;
             }
         }
-        if (lane < 8) tag[row * 8 + lane] = kp[(long)(PG - 1) * k_st + lane];
-        wave_lds_sync();
-        for (int d = lane; d < D; d += kWave) {
-            float acc = 0.f;
-            for (int t = 0; t < PG; ++t) acc = __fadd_rn(acc, L.dc[t][d]);
-            const float m = __fdiv_rn(acc, (float)PG);
-            L.mu[d] = m;
-            for (int t = 0; t < PG; ++t) L.dc[t][d] = __fsub_rn(L.dc[t][d], m);
-        }
-        wave_lds_sync();
+        // the same of page g of the wave, wave-uniform
+        auto page_row = [&](int g) { return readlane64(rwl, g * PG); };
+        auto page_k = [&](int g) { return reinterpret_cast<const uint16_t*>(readlane64(reinterpret_cast<long>(kpl), g * PG)); };
+        // the page's tokens of channels 2 l, 2 l + 1 of group k, minus their
+        // mean (a sequential sum over t; 1 / PG is a power of two)
+        auto centred = [&](const uint16_t* p, int k, float (&x)[PG][2], float (&mu)[2]) {
+            uint32_t w[PG];
+#pragma unroll
+            for (int t = 0; t < PG; ++t) w[t] = ((global_u32)(p + (long)t * k_st + 128 * k))[cl];
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int t = 0; t < PG; ++t) { a = __fadd_rn(a, bf16lo(w[t])); b = __fadd_rn(b, bf16hi(w[t])); }
+            mu[0] = __fmul_rn(a, 1.f / PG);
+            mu[1] = __fmul_rn(b, 1.f / PG);
+#pragma unroll
+            for (int t = 0; t < PG; ++t) {
+                x[t][0] = __fsub_rn(bf16lo(w[t]), mu[0]);
+                x[t][1] = __fsub_rn(bf16hi(w[t]), mu[1]);
+            }
+        };
 
-        // gram on the matrix core: Gm[i][j] = sum_d dc[i][d] dc[j][d], in
-        // 16 x 16 blocks (bi, bj) of the PG x PG matrix
-        {
-            const int i = lane & 15, kq = lane >> 4;
+        // ---- gram on the matrix core, Gm[i][j] = sum_d dc[i][d] dc[j][d], one
+        // page after the other, in 16 x 16 blocks (bi, bj)
+        const int i16 = lane & 15, kq = lane >> 4;
+        v4f gm[GW][NB16][NB16];
+#pragma unroll
+        for (int g = 0; g < GW; ++g) {
+#pragma unroll
+            for (int bi = 0; bi < NB16; ++bi)
+#pragma unroll
+                for (int bj = 0; bj < NB16; ++bj) gm[g][bi][bj] = v4f{0.f, 0.f, 0.f, 0.f};
+            const uint16_t* kp = page_k(g);
+            if (kp == nullptr) continue;
 #pragma unroll 1
-            for (int bi = 0; bi < PG / 16; ++bi)
+            for (int k = 0; k < NK; ++k) {
+                float x[PG][2], mu[2];
+                centred(kp, k, x, mu);
+#pragma unroll 1
+                for (int wi = 0; wi < NWIN; ++wi) {
+                    const int at = 2 * lane - WCH * wi;
+                    if (at >= 0 && at < WCH)
 #pragma unroll
-                for (int bj = 0; bj < PG / 16; ++bj) {
-                    v4f g = {0.f, 0.f, 0.f, 0.f};
-                    for (int s = 0; s < D / 4; ++s) {
-                        const float a = L.dc[16 * bi + i][4 * s + kq];
-                        const float b = L.dc[16 * bj + i][4 * s + kq];
-                        g = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, g, 0, 0, 0);
+                        for (int t = 0; t < PG; ++t)
+                            *reinterpret_cast<float2*>(&L.dc[t][at]) = make_float2(x[t][0], x[t][1]);
+                    wave_lds_sync();
+#pragma unroll 4
+                    for (int s = 0; s < WCH / 4; ++s) {
+                        float a[NB16];
+#pragma unroll
+                        for (int bi = 0; bi < NB16; ++bi) a[bi] = L.dc[16 * bi + i16][4 * s + kq];
+#pragma unroll
+                        for (int bi = 0; bi < NB16; ++bi)
+#pragma unroll
+                            for (int bj = 0; bj < NB16; ++bj)
+                                gm[g][bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[bi], a[bj], gm[g][bi][bj], 0, 0, 0);
                     }
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) L.A[16 * bi + 4 * kq + v][16 * bj + i] = g[v];
+                    wave_lds_sync();
                 }
+            }
         }
+        // lane (kq, i) holds rows 4 kq .. 4 kq + 3 of column i of each block;
+        // exchange so that each lane holds all PG rows of its own column
+        float A[PG], U[PG], diag = 0.f;
+#pragma unroll
+        for (int bi = 0; bi < NB16; ++bi)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                uint32_t r[4];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) r[x] = __float_as_uint(gm[x / NB16][bi][x % NB16][v]);
+                const auto s02 = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+                const auto s13 = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+                const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+                const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+                A[16 * bi + v] = __uint_as_float(s01[0]);
+                A[16 * bi + 4 + v] = __uint_as_float(s01[1]);
+                A[16 * bi + 8 + v] = __uint_as_float(s23[0]);
+                A[16 * bi + 12 + v] = __uint_as_float(s23[1]);
+            }
+        static_for<0, PG>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            U[i] = pick_lane<PG, i>(1.f, 0.f);
+            diag = pick_lane<PG, i>(A[i], diag);
+        });
+        jacobi<PG>(A, U, diag, L.cs[pg], lane);
         wave_lds_sync();
-        jacobi<PG>(L);
-        select_top8<PG>(L);
-        pack_page<D, PG>(L, row, S);
+        // ---- ascending ranks; the 8 largest: columns, singular values --------
+        {
+            // order-preserving key; NaN (a page with non-finite keys) lowest, ties by column
+            const uint32_t key = f2u(diag == diag ? diag + 0.f : -INFINITY);
+            L.top.lam[lane] = key;
+            wave_lds_sync();
+            int rank = 0;
+#pragma unroll
+            for (int m = 0; m < PG; m += 4) {
+                const uint4 l4 = *reinterpret_cast<const uint4*>(&L.top.lam[lane - j + m]);
+                const uint32_t lk[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rank += lk[e] < key + ((uint32_t)(m + e - j) >> 31) ? 1 : 0;
+            }
+            if (rank >= PG - BD_RNK) {
+                const int r = rank - (PG - BD_RNK);
+                const float s8 = __fsqrt_rn(fmaxf(diag, 1e-10f));
+                L.top.s8[pg][r] = s8;
+                L.top.y8[pg][r] = __fdiv_rn(1.f, s8);
+            }
+            L.top.lam[lane] = (uint32_t)rank;        // (every key has been read)
+            wave_lds_sync();
+#pragma unroll
+            for (int m = 0; m < PG; m += 4) {
+                const uint4 l4 = *reinterpret_cast<const uint4*>(&L.top.lam[lane - j + m]);
+                const uint32_t lk[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (lk[e] >= PG - BD_RNK) L.top.u[pg][lk[e] - (PG - BD_RNK)][j] = U[m + e];
+            }
+            wave_lds_sync();
+        }
+        // ---- coefficients: this lane owns token j of page pg ------------------
+        {
+            if (kpl != nullptr) {
+                float C[BD_RNK], am = 0.f;
+#pragma unroll
+                for (int r = 0; r < BD_RNK; ++r) {
+                    C[r] = __fmul_rn(L.top.u[pg][r][j], L.top.s8[pg][r]);
+                    am = fmaxf(am, fabsf(C[r]));
+                }
+                const float csc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f), y = __fdiv_rn(1.f, csc);
+                uint32_t wd[2] = {0u, 0u};
+#pragma unroll
+                for (int r = 0; r < BD_RNK; ++r) {
+                    const int q = (int)fminf(fmaxf(rintf(div_by(C[r], csc, y)), -127.f), 127.f);
+                    wd[r >> 2] |= (uint32_t)(q & 255) << (8 * (r & 3));
+                }
+                *reinterpret_cast<uint2*>(S.c8 + rwl * S.sc8 + j * BD_RNK) = make_uint2(wd[0], wd[1]);
+                reinterpret_cast<uint16_t*>(S.cs + rwl * S.scs)[j] = f32_to_bf16(csc);
+                if (j < 8) tag[rwl * 8 + j] = kpl[(long)(PG - 1) * k_st + j];
+            }
+        }
+        // ---- basis and centroid, one page after the other ---------------------
+#pragma unroll 1
+        for (int g = 0; g < gpw; ++g) {
+            const uint16_t* kp = page_k(g);
+            if (kp == nullptr) continue;
+            const long rw = page_row(g);
+            float V[NK][2][BD_RNK], mu[NK][2];
+#pragma unroll
+            for (int k = 0; k < NK; ++k) {
+                float x[PG][2];
+                centred(kp, k, x, mu[k]);
+#pragma unroll
+                for (int r = 0; r < BD_RNK; ++r) {
+                    float a = 0.f, b = 0.f;                 // sequential over t
+#pragma unroll
+                    for (int t = 0; t < PG; ++t) {
+                        const float u = L.top.u[g][r][t];
+                        a = __fadd_rn(a, __fmul_rn(x[t][0], u));
+                        b = __fadd_rn(b, __fmul_rn(x[t][1], u));
+                    }
+                    const float s8 = L.top.s8[g][r], y8 = L.top.y8[g][r];
+                    V[k][0][r] = div_by(a, s8, y8);
+                    V[k][1][r] = div_by(b, s8, y8);
+                }
+            }
+            // Maxima over the channels of the 8 columns and the centroid.  Two
+            // pair swaps fold the columns into one lane row each (lane row x of
+            // m[0]: column x' = 2 (x & 1) + (x >> 1), of m[1]: 4 + x'), then each
+            // row reduces; its lanes 0, 1, 2 turn the two columns' and the
+            // centroid's maximum into a scale, read back lane by lane.
+            float m[BD_RNK], mm = 0.f;
+#pragma unroll
+            for (int k = 0; k < NK; ++k) mm = fmaxf(mm, fmaxf(fabsf(mu[k][0]), fabsf(mu[k][1])));
+            mm = wave_max(mm);
+#pragma unroll
+            for (int r = 0; r < BD_RNK; ++r) {
+                m[r] = 0.f;
+#pragma unroll
+                for (int k = 0; k < NK; ++k) m[r] = fmaxf(m[r], fmaxf(fabsf(V[k][0][r]), fabsf(V[k][1][r])));
+            }
+#pragma unroll
+            for (int r = 0; r < BD_RNK / 2; ++r) {            // columns 2 r (lower half), 2 r + 1
+                const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[2 * r]), __float_as_uint(m[2 * r + 1]), false, false);
+                m[r] = fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+            }
+#pragma unroll
+            for (int r = 0; r < BD_RNK / 4; ++r) {
+                const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(m[2 * r]), __float_as_uint(m[2 * r + 1]), false, false);
+                float x = fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+                x = fmaxf(x, row_ror<8>(x));
+                x = fmaxf(x, row_ror<4>(x));
+                x = fmaxf(x, row_ror<2>(x));
+                m[r] = fmaxf(x, row_ror<1>(x));
+            }
+            const float am = i16 == 0 ? m[0] : i16 == 1 ? m[1] : mm;
+            const float sc = fmaxf(__fdiv_rn(am, i16 < 2 ? 7.f : 127.f), 1e-8f);
+            const float ys = __fdiv_rn(1.f, sc);
+            if (i16 < 2)
+                reinterpret_cast<uint16_t*>(S.vs + rw * S.svs)[4 * i16 + 2 * (kq & 1) + (kq >> 1)] = f32_to_bf16(sc);
+            if (lane == 2) *reinterpret_cast<uint16_t*>(S.mus + rw * S.smus) = f32_to_bf16(sc);
+            auto of_lane = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+            uint8_t* vrow = S.v4 + rw * S.sv4;
+#pragma unroll
+            for (int r = 0; r < BD_RNK; ++r) {
+                const int at = 16 * (((r & 1) << 1) | ((r >> 1) & 1)) + (r >> 2);   // the lane of column r
+                const float b = of_lane(sc, at), y = of_lane(ys, at);
+#pragma unroll
+                for (int k = 0; k < NK; ++k) {
+                    const int lo = (int)fminf(fmaxf(rintf(div_by(V[k][0][r], b, y)), -8.f), 7.f);
+                    const int hi = (int)fminf(fmaxf(rintf(div_by(V[k][1][r], b, y)), -8.f), 7.f);
+                    if (own) vrow[r * (D / 2) + 64 * k + lane] = (uint8_t)((lo & 15) | ((hi & 15) << 4));
+                }
+            }
+            const float b = of_lane(sc, 2), y = of_lane(ys, 2);
+#pragma unroll
+            for (int k = 0; k < NK; ++k) {
+                const int lo = (int)fminf(fmaxf(rintf(div_by(mu[k][0], b, y)), -127.f), 127.f);
+                const int hi = (int)fminf(fmaxf(rintf(div_by(mu[k][1], b, y)), -127.f), 127.f);
+                if (own)
+                    reinterpret_cast<uint16_t*>(S.mu + rw * S.smu)[64 * k + lane] =
+                        (uint16_t)((lo & 255) | ((hi & 255) << 8));
+            }
+        }
+        wave_lds_sync();                                     // the columns are read before the next gram
     }
 }
 
@@ -469,12 +708,13 @@ template <int D, int PG>
 static int bd_launch(const uint16_t* kc, const uint64_t* k_layers, long k_sb, long k_st, long k_sh,
                      int NB, const int* blocks, const int* count, int n_blocks, int n_kv,
                      int n_layers, long layer_rows, const SlabRows& S, uint16_t* tag, hipStream_t st) {
-    constexpr int nw = bd_waves<D, PG>();
     const long items = (long)n_blocks * n_kv * n_layers;
-    const long grid = std::min((items + nw - 1) / nw, BD_MAX_GRID);
-    hipLaunchKernelGGL((rki4_build_kernel<D, PG>), dim3((unsigned)grid), dim3(nw * kWave), 0, st,
-                       kc, k_layers, k_sb, k_st, k_sh, NB, blocks, count, n_blocks, n_kv,
-                       n_layers, layer_rows, S, tag);
+    // few items: one page per wave, on as many SIMDs as there are items
+    const int gpw = items <= BD_SPREAD ? 1 : kWave / PG;
+    const long grid = std::min((items + 4 * gpw - 1) / (4 * gpw), BD_MAX_GRID);
+    hipLaunchKernelGGL((rki4_build_kernel<D, PG>), dim3((unsigned)grid), dim3(4 * kWave), 0, st, kc,
+                       k_layers, k_sb, k_st, k_sh, NB, blocks, count, n_blocks, n_kv, n_layers,
+                       layer_rows, S, tag, gpw);
     return check_launch("rki4_build_kernel");
 }
 #define BD_DISPATCH(HD, PGV, ...)                                              \
