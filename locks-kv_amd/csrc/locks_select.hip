@@ -16,16 +16,17 @@
 // MI355X design.  At 1M context one (request, kv head) has 65536 pages and
 // bs=1 GLM has only two such groups, so a one-workgroup-per-group selector
 // would read 4 MB of score_h through a single CU.  Instead:
-//   sel_chunk_kernel  (grid: page chunks x kv heads x requests)
-//       forms hm from the scorer's per-chunk maxima, combines its 2048-page
-//       chunk, writes `score`, prefills its slice of page_table with -1, and
-//       emits the chunk's local top-b candidates (the total order restricted
-//       to a chunk keeps every globally kept page of that chunk) in ascending
-//       page order.  When one chunk covers the whole row it finishes the
-//       selection itself (one launch).
-//   sel_finish_kernel (grid: kv heads x requests)
-//       gathers the <= b candidates of every chunk into LDS, radix-selects
-//       the exact b-th largest key and compacts the kept pages.
+//   sel_row_kernel     (grid: kv heads x requests; rows of at most 8192 pages)
+//       combines the row and selects from keys held in registers, one launch.
+//   sel_chunk2_kernel  (grid: page chunks x kv heads x requests)
+//       forms hm from the scorer's per-chunk maxima, combines its 1024- or
+//       2048-page chunk, writes `score`, prefills its slice of page_table with
+//       -1, and emits the chunk's local top-b candidates (the total order
+//       restricted to a chunk keeps every globally kept page of that chunk) in
+//       ascending page order; sel_band_kernel emits them for large budgets.
+//   sel_finish2_kernel (grid: kv heads x requests)
+//       gathers the candidates of every chunk, radix-selects the exact b-th
+//       largest key and compacts the kept pages.
 // (Folding the finish into the last-arriving chunk needs an agent-scope
 // release fence, which on MI355X writes back the XCD's dirty L2 and measured
 // slower than the second launch.)
@@ -39,9 +40,6 @@
 namespace locks {
 
 constexpr int SEL_CH = 2048;       // pages per chunk workgroup
-constexpr int SEL_BLK = 512;       // threads per chunk workgroup
-constexpr int FIN_BLK = 1024;      // threads of the finishing workgroup
-constexpr int FIN_CAP = 6144;      // candidates held in LDS by the finisher
 constexpr int FIN_MAXZ = 1024;     // chunks per row the finisher can index
 
 // ---------------------------------------------------------------------------
@@ -210,24 +208,17 @@ __device__ __forceinline__ float chunk_max(const float* __restrict__ p, int n) {
     return m;
 }
 
-__device__ __forceinline__ void fill_all_pages(int* row, int n_pages, int MP, bool pad) {
-    for (int i = threadIdx.x; i < MP; i += blockDim.x) {
-        if (i < n_pages) row[i] = i;
-        else if (pad) row[i] = -1;
-    }
-}
-
 // Finish one row from the chunk candidates (ascending page order per chunk):
 // exact b-th largest key over all candidates, ordered emission, sink/window.
-// LDS arguments: offs[FIN_MAXZ+1], lkey/lpage[cap] (more candidates spill to
-// the global workspace), hist[256], s3[4], wsum.
+// The candidates are gathered in the global workspace (more of them than
+// sel_finish2_kernel holds in registers).  LDS arguments: offs[FIN_MAXZ+1],
+// hist[256], s3[4], wsum.
 template <int BLK>
 __device__ void finish_row(long rk, int n_pages, int n_sel_hi, int n_sink, int b, int MP, int Z1,
                            int* __restrict__ trow, int* __restrict__ cnt_out,
                            const uint32_t* __restrict__ cand_key, const int* __restrict__ cand_page,
                            const int* __restrict__ cand_cnt, uint32_t* __restrict__ spill_key,
-                           int* __restrict__ spill_page, int* offs, uint32_t* lkey, int* lpage,
-                           int* hist, int* s3, int* wsum, int cap = FIN_CAP) {
+                           int* __restrict__ spill_page, int* offs, int* hist, int* s3, int* wsum) {
     constexpr int NWV = BLK / kWave;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     {
@@ -244,8 +235,8 @@ __device__ void finish_row(long rk, int n_pages, int n_sel_hi, int n_sink, int b
         lds_barrier();
     }
     const int N = offs[Z1];
-    uint32_t* kk = (N <= cap) ? lkey : spill_key + rk * (long)MP;
-    int* pp = (N <= cap) ? lpage : spill_page + rk * (long)MP;
+    uint32_t* kk = spill_key + rk * (long)MP;
+    int* pp = spill_page + rk * (long)MP;
     for (int zz = wave; zz < Z1; zz += NWV) {                 // chunk order == page order
         const int o = offs[zz], c = offs[zz + 1] - o;
         const uint32_t* sk = cand_key + (rk * Z1 + zz) * (long)SEL_CH;
@@ -266,7 +257,7 @@ __device__ void finish_row(long rk, int n_pages, int n_sel_hi, int n_sink, int b
             }
         }
     }
-    __syncthreads();                    // candidates may be in global spill memory
+    __syncthreads();                    // the candidates are in global memory
     const uint32_t tau = block_kth_largest<BLK>(kk, N, b, hist, s3);
     const int nsel_w = emit_topk<BLK>(kk, N, b, tau, [&](int i) { return pp[i]; },
                                       trow + n_sink, nullptr, wsum);
@@ -503,7 +494,9 @@ __device__ int reg_emit(const uint32_t (&key)[E], const bool (&val)[E], const Ra
 // (request, kv head) does combine, exact top-b and the page table in one
 // launch.  Thread t owns pages [E t, E t + E) (contiguous, so one packed
 // block scan orders the emission); the keys stay in registers; the radix
-// select runs 12 + 12 + 8-bit MSD passes over an LDS histogram.
+// select runs 12 + 12 + 8-bit MSD passes over an LDS histogram.  (Short rows
+// on 256- or 512-thread workgroups with 1024-bin histograms measured the same
+// step: 50.3 / 50.4 us for two layers at 32K.)
 // ---------------------------------------------------------------------------
 constexpr int ROW_BLK = 1024;
 constexpr int ROW_NW = ROW_BLK / kWave;
@@ -512,7 +505,16 @@ constexpr int ROW_NW = ROW_BLK / kWave;
 // 20.5 us; G = 16: 44.8 vs 25.7 us).
 constexpr int ROW_MAXP = 8 * ROW_BLK;
 
-template <int E, int HB = (E <= 8) ? 8 : 4>
+// Rows of score_h and page_table start 4-byte aligned when max_pages is not a
+// multiple of 4: vector accesses of that alignment.
+typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef int i4a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// ROW: the row's length -- 0: a multiple of 4 pages; 1: any other of at least
+// 4; 2: at most 3.  (As run-time branches around the loads the other two made
+// every load wait at a join: step 129 -> 142 us at 128K.)
+template <int E, int HB, int ROW>
 __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     const float* __restrict__ score_h, const float* __restrict__ pmax, int Zs,
     const int* __restrict__ npg, const int* __restrict__ nsh, const int* __restrict__ bfix,
@@ -559,16 +561,31 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
                 // unconditional (clamped) loads: surplus heads / pages are
                 // never combined or kept, and a guarded load would make the
                 // compiler wait for it before the page maxima are requested
-                const int g = min(g0 + j, G - 1), p = min(p0 + 4 * v, MP - 4);
-                xv[j][v] = *reinterpret_cast<const float4*>(shb + (long)g * MP + p);
+                const float* row = shb + (long)min(g0 + j, G - 1) * MP;
+                const int p = p0 + 4 * v;
+                if constexpr (ROW == 0) {
+                    xv[j][v] = *reinterpret_cast<const float4*>(row + min(p, MP - 4));
+                } else if constexpr (ROW == 1) {
+                    const f4a4 x = *reinterpret_cast<const f4a4*>(row + min(p, MP - 4));
+                    xv[j][v] = make_float4(x[0], x[1], x[2], x[3]);
+                } else {
+                    xv[j][v] = make_float4(row[min(p, MP - 1)], row[min(p + 1, MP - 1)], row[min(p + 2, MP - 1)],
+                                           row[MP - 1]);
+                }
             }
+    };
+    // A row of 4 k + 1 .. 3 pages: the one thread whose vector runs past it
+    // loaded the row's last four and takes its pages from the vector's end.
+    auto tail_shift = [&](float (&x)[4], int p) {
+        const int sh = p < MP ? p - (MP - 4) : 0;
+        x[0] = sh == 1 ? x[1] : sh == 2 ? x[2] : sh == 3 ? x[3] : x[0];
+        x[1] = sh == 1 ? x[2] : sh >= 2 ? x[3] : x[1];
+        x[2] = sh >= 1 ? x[3] : x[2];
     };
     load_batch(0);
     if (combine == 0) {
         if (wave < G) {
-            float m = -INFINITY;
-            m = chunk_max(pmax + (rk * 16 + wave) * Zs, Zs);
-            m = wave_max(m);
+            const float m = wave_max(chunk_max(pmax + (rk * 16 + wave) * Zs, Zs));
             if (lane == 0) hm[wave] = m;
         }
         lds_barrier();
@@ -589,7 +606,8 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
                 const float h = hm[min(g0 + j, G - 1)];
 #pragma unroll
                 for (int v = 0; v < E / 4; ++v) {
-                    const float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
+                    float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
+                    if constexpr (ROW == 1) tail_shift(x4, p0 + 4 * v);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float t = __expf(x4[i] - h);
@@ -603,7 +621,8 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
                 const int g = g0 + j;
 #pragma unroll
                 for (int v = 0; v < E / 4; ++v) {
-                    const float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
+                    float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
+                    if constexpr (ROW == 1) tail_shift(x4, p0 + 4 * v);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float mx = (g == 0) ? x4[i] : fmaxf(acc[4 * v + i], x4[i]);
@@ -617,7 +636,7 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     if (p0 + E <= pend) {
 #pragma unroll
         for (int v = 0; v < E / 4; ++v)
-            *reinterpret_cast<float4*>(srow + p0 + 4 * v) = make_float4(acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]);
+            *reinterpret_cast<f4a4*>(srow + p0 + 4 * v) = f4a4{acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]};
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e)
@@ -641,7 +660,7 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     const int cnt = n_sink + b + (n_pages - n_sel_hi);
     if (p0 >= cnt && p0 + E <= MP) {                      // padding only
 #pragma unroll
-        for (int v = 0; v < E / 4; ++v) *reinterpret_cast<int4*>(trow + p0 + 4 * v) = make_int4(-1, -1, -1, -1);
+        for (int v = 0; v < E / 4; ++v) *reinterpret_cast<i4a4*>(trow + p0 + 4 * v) = i4a4{-1, -1, -1, -1};
     } else if (p0 < n_sink || p0 + E > n_sink + b) {     // not only kept slots
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -669,164 +688,6 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     const RadixSel rs = reg_kth_largest<ROW_BLK, E>(key, val, b, hist, wtot, s3, mk_bound);
     // wsum is not used again: no closing barrier after the emission scan
     reg_emit<ROW_BLK, E, false>(key, val, rs, wsum, [&](int pos, int e) { trow[n_sink + pos] = p0 + e; });
-}
-
-// ---------------------------------------------------------------------------
-// chunk kernel
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(SEL_BLK) void sel_chunk_kernel(
-    const float* __restrict__ score_h, const float* __restrict__ pmax, int Zs,
-    const int* __restrict__ npg, const int* __restrict__ nsh, const int* __restrict__ bfix,
-    float* __restrict__ score, int* __restrict__ page_table, int* __restrict__ page_cnt,
-    uint32_t* __restrict__ cand_key, int* __restrict__ cand_page, int* __restrict__ cand_cnt,
-    int n_sink, int MP, int G, int combine)
-{
-    const int z = blockIdx.x, kh = blockIdx.y, r = blockIdx.z;
-    const int n_kv = gridDim.y, Z1 = gridDim.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const long rk = (long)r * n_kv + kh;
-    const int n_pages = min(npg[r], MP);
-    const int n_sel_hi = min(nsh[r], MP);
-    const int n_sel = n_sel_hi - n_sink;
-    const bool keep_all = n_sel <= 1;
-    int b = bfix[r];
-    b = max(1, min(b, max(n_sel, 1)));
-    const bool final_mode = (Z1 == 1);
-    const int c0 = z * SEL_CH;
-    const int c1 = min(c0 + SEL_CH, MP);
-
-    __shared__ float hm[16];
-    __shared__ uint32_t keys[SEL_CH];
-    __shared__ int hist[256];
-    __shared__ int s3[4];
-    __shared__ int wsum[SEL_BLK / kWave + 1];
-
-    int* trow = page_table + rk * (long)MP;
-    if (!final_mode) {
-        for (int i = c0 + tid; i < c1; i += SEL_BLK) trow[i] = -1;
-    }
-
-    // ---- issue every score_h load of this thread first (4 pages x G rows)
-    const float* shb = score_h + rk * (long)G * MP;
-    const int pend = min(c1, max(n_sel_hi, c0));
-    constexpr int SEL_E = SEL_CH / SEL_BLK;
-    float x[SEL_E][16];
-#pragma unroll
-    for (int e = 0; e < SEL_E; ++e) {
-        const int p = c0 + tid + e * SEL_BLK;
-#pragma unroll
-        for (int g = 0; g < 16; ++g)
-            x[e][g] = (g < G && p < pend) ? shb[(long)g * MP + p] : 0.f;
-    }
-
-    // ---- per-head page max from the scorer's chunk maxima ("nrm") --------
-    if (combine == 0) {
-        for (int g = wave; g < G; g += SEL_BLK / kWave) {
-            float m = -INFINITY;
-            m = chunk_max(pmax + (rk * 16 + g) * Zs, Zs);
-            m = wave_max(m);
-            if (lane == 0) hm[g] = m;
-        }
-        lds_barrier();
-    }
-
-    // ---- combine: score[p] for p < nsh, keys for the selectable slice ----
-#pragma unroll
-    for (int e = 0; e < SEL_E; ++e) {
-        const int p = c0 + tid + e * SEL_BLK;
-        if (p >= pend) continue;
-        float acc;
-        if (combine == 0) {
-            acc = 0.f;
-#pragma unroll
-            for (int g = 0; g < 16; ++g)
-                if (g < G) acc += __expf(x[e][g] - hm[g]);
-        } else {
-            acc = x[e][0];
-#pragma unroll
-            for (int g = 1; g < 16; ++g)
-                if (g < G) acc = fmaxf(acc, x[e][g]);
-        }
-        score[rk * (long)MP + p] = acc;
-        keys[p - c0] = f2u(acc);
-    }
-    lds_barrier();
-
-    const int lo_c = min(max(n_sink, c0), c1) - c0;       // selectable slice of
-    const int hi_c = max(min(n_sel_hi, c1), c0) - c0;     // this chunk, local idx
-    const int n_loc = max(hi_c - lo_c, 0);
-
-    if (final_mode) {
-        // the whole row lives in this chunk: finish here
-        if (keep_all || b >= n_sel) {
-            fill_all_pages(trow, max(n_pages, 0), MP, true);
-            if (tid == 0) page_cnt[rk] = max(n_pages, 0);
-            return;
-        }
-        const uint32_t tau = block_kth_largest<SEL_BLK>(keys + lo_c, n_loc, b, hist, s3);
-        const int nsel_w = emit_topk<SEL_BLK>(keys + lo_c, n_loc, b, tau,
-                                              [&](int i) { return n_sink + i; },
-                                              trow + n_sink, nullptr, wsum);
-        const int cnt = n_sink + nsel_w + (n_pages - n_sel_hi);
-        for (int i = tid; i < MP; i += SEL_BLK) {
-            if (i < n_sink) trow[i] = i;
-            else if (i >= n_sink + nsel_w && i < cnt) trow[i] = n_sel_hi + (i - n_sink - nsel_w);
-            else if (i >= cnt) trow[i] = -1;
-        }
-        if (tid == 0) page_cnt[rk] = cnt;
-        return;
-    }
-
-    // ---- multi-chunk: emit this chunk's local top-min(b, n_loc) ----------
-    uint32_t* ck = cand_key + (rk * Z1 + z) * (long)SEL_CH;
-    int* cp = cand_page + (rk * Z1 + z) * (long)SEL_CH;
-    int ncand = 0;
-    if (!keep_all && n_loc > 0) {
-        const int k_loc = min(b, n_loc);
-        uint32_t tau = 0u;   // k_loc == n_loc: every key >= 0 is kept
-        if (k_loc < n_loc) tau = block_kth_largest<SEL_BLK>(keys + lo_c, n_loc, k_loc, hist, s3);
-        const int base = c0 + lo_c;
-        ncand = emit_topk<SEL_BLK>(keys + lo_c, n_loc, k_loc, tau,
-                                   [&](int i) { return base + i; }, cp, ck, wsum);
-    }
-    if (tid == 0) cand_cnt[rk * Z1 + z] = ncand;
-}
-
-// ---------------------------------------------------------------------------
-// finishing kernel (multi-chunk rows)
-// ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
-// finishing kernel (rows spanning several chunks)
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(FIN_BLK) void sel_finish_kernel(
-    const int* __restrict__ npg, const int* __restrict__ nsh, const int* __restrict__ bfix,
-    int* __restrict__ page_table, int* __restrict__ page_cnt,
-    const uint32_t* __restrict__ cand_key, const int* __restrict__ cand_page,
-    const int* __restrict__ cand_cnt, uint32_t* __restrict__ spill_key, int* __restrict__ spill_page,
-    int n_sink, int MP, int Z1)
-{
-    const int kh = blockIdx.y, r = blockIdx.z;
-    const long rk = (long)r * gridDim.y + kh;
-    const int n_pages = min(npg[r], MP);
-    const int n_sel_hi = min(nsh[r], MP);
-    const int n_sel = n_sel_hi - n_sink;
-    int b = bfix[r];
-    b = max(1, min(b, max(n_sel, 1)));
-    int* trow = page_table + rk * (long)MP;
-    if (n_sel <= 1 || b >= n_sel) {
-        for (int i = threadIdx.x; i < max(n_pages, 0); i += FIN_BLK) trow[i] = i;
-        if (threadIdx.x == 0) page_cnt[rk] = max(n_pages, 0);
-        return;
-    }
-    __shared__ int offs[FIN_MAXZ + 1];
-    __shared__ uint32_t lkey[FIN_CAP];
-    __shared__ int lpage[FIN_CAP];
-    __shared__ int hist[256];
-    __shared__ int s3[4];
-    __shared__ int wsum[FIN_BLK / kWave + 1];
-    finish_row<FIN_BLK>(rk, n_pages, n_sel_hi, n_sink, b, MP, Z1, trow, page_cnt + rk, cand_key,
-                        cand_page, cand_cnt, spill_key, spill_page, offs, lkey, lpage, hist, s3,
-                        wsum);
 }
 
 // ---------------------------------------------------------------------------
@@ -877,9 +738,10 @@ __global__ __launch_bounds__(C2_BLK) void sel_chunk2_kernel(
     float2 xv[GL];
 #pragma unroll
     for (int g = 0; g < GL; ++g) {                       // clamped, unconditional (see the row kernel)
-        if constexpr (E == 2)
-            xv[g] = *reinterpret_cast<const float2*>(shb + (long)min(g, G - 1) * MP + min(p0, MP - 2));
-        else
+        if constexpr (E == 2) {
+            const f2a4 x = *reinterpret_cast<const f2a4*>(shb + (long)min(g, G - 1) * MP + min(p0, MP - 2));
+            xv[g] = make_float2(p0 == MP - 1 ? x[1] : x[0], x[1]);   // an odd row's last page: the pair's second
+        } else
             xv[g] = make_float2(shb[(long)min(g, G - 1) * MP + min(p0, MP - 1)], 0.f);
     }
     int* trow = page_table + rk * (long)MP;
@@ -930,7 +792,7 @@ __global__ __launch_bounds__(C2_BLK) void sel_chunk2_kernel(
     float* srow = score + rk * (long)MP;
     if constexpr (E == 2) {
         if (p0 + E <= pend) {
-            *reinterpret_cast<float2*>(srow + p0) = make_float2(acc[0], acc[E - 1]);
+            *reinterpret_cast<f2a4*>(srow + p0) = f2a4{acc[0], acc[E - 1]};
         } else {
 #pragma unroll
             for (int e = 0; e < E; ++e)
@@ -1181,8 +1043,7 @@ __global__ __launch_bounds__(F2_BLK) void sel_finish2_kernel(
     const int N = offs[Z1];
     if (N > F2_CAP) {                   // more candidates than registers: global spill
         finish_row<F2_BLK>(rk, n_pages, n_sel_hi, n_sink, b, MP, Z1, trow, page_cnt + rk, cand_key,
-                           cand_page, cand_cnt, spill_key, spill_page, offs, nullptr, nullptr, hist,
-                           s3, wsum, 0);
+                           cand_page, cand_cnt, spill_key, spill_page, offs, hist, s3, wsum);
         return;
     }
     if (N <= F2_BLK * 4)
@@ -1289,27 +1150,36 @@ extern "C" int32_t locks_select_nrm_topb(
     // The row kernel also serves rows of one chunk or less: against the
     // single-chunk kernel it measured GLM 16K 1.225 -> 1.083 ms and 32K
     // 1.327 -> 1.104 ms per step
-    if (max_pages <= ROW_MAXP && max_pages % 4 == 0 &&
-        (long)G * max_pages <= SEL_ROW_MAX_GP) {
-#define ROW_LAUNCH(EV, HBV)                                                                \
-        hipLaunchKernelGGL((sel_row_kernel<EV, HBV>), dim3(n_kv, n_req), dim3(ROW_BLK), 0, st, score_h, \
+    // Both routes take rows of any length.  A page count that is not a multiple
+    // of 4 took a 512-thread chunk kernel and, past 2048 pages, a second launch:
+    // step of two layers at 50001 tokens 93 -> 57 us, 20001 65 -> 52, 300001
+    // 132 -> 99 (10 % budget 246 -> 162), G = 16 at 150100 104 -> 69.
+    if (max_pages <= ROW_MAXP && (long)G * max_pages <= SEL_ROW_MAX_GP) {
+#define ROW_LAUNCH(EV, HBV, RV)                                                                \
+        hipLaunchKernelGGL((sel_row_kernel<EV, HBV, RV>), dim3(n_kv, n_req), dim3(ROW_BLK), 0, st, score_h, \
                            page_max, score_chunks, n_pages, n_sel_hi, b_fix, score, page_table, \
                            page_cnt, n_sink, max_pages, G, combine)
         // heads per load batch: no clamped duplicate loads for one head (MLA)
         // or groups of at most 4 (Llama G = 4: 16 -> 8 loads per thread)
-        if (max_pages <= 4 * ROW_BLK) {
-            if (G == 1) ROW_LAUNCH(4, 1);
-            else if (G <= 4) ROW_LAUNCH(4, 4);
-            else ROW_LAUNCH(4, 8);
+#define ROW_LAUNCH_G(EV, RV)                                                                   \
+        do {                                                                                   \
+            if (G == 1) ROW_LAUNCH(EV, 1, RV);                                                 \
+            else if (G <= 4) ROW_LAUNCH(EV, 4, RV);                                            \
+            else ROW_LAUNCH(EV, 8, RV);                                                        \
+        } while (0)
+        if (max_pages < 4) ROW_LAUNCH(4, 8, 2);
+        else if (max_pages <= 4 * ROW_BLK) {
+            if (max_pages % 4 == 0) ROW_LAUNCH_G(4, 0);
+            else ROW_LAUNCH_G(4, 1);
         } else {
-            if (G == 1) ROW_LAUNCH(8, 1);
-            else if (G <= 4) ROW_LAUNCH(8, 4);
-            else ROW_LAUNCH(8, 8);
+            if (max_pages % 4 == 0) ROW_LAUNCH_G(8, 0);
+            else ROW_LAUNCH_G(8, 1);
         }
+#undef ROW_LAUNCH_G
 #undef ROW_LAUNCH
         return check_launch("sel_row_kernel");
     }
-    if (Z1 > 1 && max_pages % 4 == 0) {
+    {
         // Local top-b lists of every chunk past the 4-per-thread finisher:
         // the histogram (band) route is faster (measured at 256K..1M with
         // b = 1638..6553: 25-36 us against 40-160 us).
@@ -1367,16 +1237,6 @@ extern "C" int32_t locks_select_nrm_topb(
         return check_launch("sel_finish2_kernel");
 #undef C2_LAUNCH
     }
-    hipLaunchKernelGGL(sel_chunk_kernel, dim3(Z1, n_kv, n_req), dim3(SEL_BLK), 0, st,
-                       score_h, page_max, score_chunks, n_pages, n_sel_hi, b_fix, score,
-                       page_table, page_cnt, cand_key, cand_page, cand_cnt, n_sink,
-                       max_pages, G, combine);
-    int rc = check_launch("sel_chunk_kernel");
-    if (rc || Z1 == 1) return rc;
-    hipLaunchKernelGGL(sel_finish_kernel, dim3(1, n_kv, n_req), dim3(FIN_BLK), 0, st,
-                       n_pages, n_sel_hi, b_fix, page_table, page_cnt, cand_key, cand_page,
-                       cand_cnt, spill_key, spill_page, n_sink, max_pages, Z1);
-    return check_launch("sel_finish_kernel");
 }
 
 extern "C" int32_t locks_derive_params(const int32_t* seq_lens, int32_t n_req, int32_t page,
