@@ -30,6 +30,23 @@ def _split_kv(kv_cache: torch.Tensor):
     return kv_cache.select(1, 0), kv_cache.select(1, 1)
 
 
+def _kv_args(kv_cache: torch.Tensor):
+    """What a kernel call takes of _split_kv's views, without making them:
+    (K address, V address or None, (block, token, head) element strides,
+    (num_blocks, page, n_kv, d))."""
+    shape, strides = kv_cache.shape, kv_cache.stride()
+    at = 0 if shape[0] == 2 and shape[1] != 2 else 1             # the dim of the two halves
+    k = kv_cache.data_ptr()
+    v = None if at == 1 and shape[1] == 1 else k + strides[at] * kv_cache.element_size()
+    n0, n1, n2, n3 = shape[:at] + shape[at + 1:]
+    sb, st, sh, _sd = strides[:at] + strides[at + 1:]
+    return k, v, (sb, st, sh), (n0, n1, n2, n3)
+
+
+_NO_V = ("ResidentVSource requires a resident V half; this cache is K-only: decode it with the DRAM "
+         "tier's source (locks.tier.TierVSource, mem variants)")
+
+
 class ResidentVSource:
     """V = the resident engine V half of kv_cache (V_SRC=0, decode.py:76-101)."""
 
@@ -38,9 +55,7 @@ class ResidentVSource:
     def __init__(self, kv_cache: torch.Tensor):
         _, v = _split_kv(kv_cache)
         if v is None:
-            raise ValueError("ResidentVSource requires a resident V half; this cache is "
-                             "K-only: decode it with the DRAM tier's source "
-                             "(locks.tier.TierVSource, mem variants)")
+            raise ValueError(_NO_V)
         self._v = v
 
     def args(self):
@@ -244,11 +259,35 @@ def sparse_paged_decode_batched(q, kv_cache, block_table, seq_lens, st, out,
     if scale is None:
         scale = st.scale
     n_req = seq_lens.shape[0]
+    pps = _pps_min(n_req, st.n_kv)
+    mc = page_cnt_bound(st)
+    if vsource is None and not FUSED_MERGE:
+        # the resident step's two launches, from addresses and strides alone
+        # (views and per-stage argument lists: 24 -> 13.5 us of host time a layer)
+        _check_out(out)
+        kp, vp, ks, (NB, page, n_kv, d) = _kv_args(kv_cache)
+        if vp is None:
+            raise ValueError(_NO_V)
+        lib, stream = _lib.load(), _lib.stream_ptr(q.device)
+        pt, cnt = st.page_table, st.page_cnt
+        pt_sr, pt_sh, _ = pt.stride()
+        q_sr, q_sh = q.stride()[:2]
+        o_sr, o_sh = out.stride()[:2]
+        parts = (st.m_part.data_ptr(), st.l_part.data_ptr(), st.acc_part.data_ptr())
+        cnt_p, cnt_s, cols, G, split = cnt.data_ptr(), cnt.stride(0), pt.shape[2], int(st.G), int(st.split)
+        _lib.check(lib.locks_decode_splitk(
+            q.data_ptr(), q_sr, q_sh, kp, *ks, vp, *ks, NB,
+            block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+            pt.data_ptr(), pt_sr, pt_sh, cols, cnt_p, cnt_s, seq_lens.data_ptr(),
+            *parts, int(n_req), n_kv, G, d, page, split, pps, mc, float(scale), stream), "decode_splitk")
+        _lib.check(lib.locks_decode_merge(
+            *parts, cnt_p, cnt_s, cols, out.data_ptr(), o_sr, o_sh,
+            1 if out.dtype == torch.float32 else 0, int(n_req), int(st.n_kv), G, st.acc_part.shape[-1], split, pps, mc,
+            stream), "decode_merge")
+        return
     k, _ = _split_kv(kv_cache)
     if vsource is None:
         vsource = ResidentVSource(kv_cache)
-    pps = _pps_min(n_req, st.n_kv)
-    mc = page_cnt_bound(st)
     if vsource.SRC_ID == 1:
         # DRAM tier (decode_cuda.py:1301-1314): split kernel with the tier's
         # source select, then the same merge

@@ -43,15 +43,14 @@ def rki4_score_only(st, layer: int, q, block_table, seq_lens, n_req: int,
     if q.dtype != torch.bfloat16 or q.stride(-1) != 1:
         raise TypeError("q must be bf16 with a contiguous head dim")
     _check_i32("block_table", block_table)
-    v4, vs, c8, cs, mu8, mus, _tag = st.layer_state(layer)
     q3 = q.view(q.shape[0], -1, st.d) if q.dim() == 2 else q
+    q_sr, q_sh = q3.stride()[:2]
     lib = _lib.load()
     _lib.check(lib.locks_score_rki4(
-        _lib.ptr(q3), q3.stride(0), q3.stride(1),
-        _lib.ptr(v4), _lib.ptr(vs), _lib.ptr(c8), _lib.ptr(cs), _lib.ptr(mu8), _lib.ptr(mus),
-        _lib.rows_arg(st), int(st.NB), _lib.ptr(block_table), block_table.stride(0), int(block_table.shape[1]),
-        _lib.ptr(st.n_sel_hi), _lib.ptr(st.score_h), int(st.max_pages),
-        _lib.ptr(st.page_max), int(st.score_chunk), int(n_req), int(st.n_kv), int(st.G),
+        q3.data_ptr(), q_sr, q_sh, *st.layer_ptrs(layer), _lib.rows_arg(st), int(st.NB),
+        block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+        st.n_sel_hi.data_ptr(), st.score_h.data_ptr(), int(st.max_pages),
+        st.page_max.data_ptr(), int(st.score_chunk), int(n_req), int(st.n_kv), int(st.G),
         int(st.d), int(st.page), float(scale), _lib.stream_ptr(q.device)), "rki4_score")
 
 
@@ -62,10 +61,10 @@ def rki4_select_only(st, n_req: int) -> None:
     lib = _lib.load()
     combine = 0 if st.combine == "nrm" else 1
     _lib.check(lib.locks_select_nrm_topb(
-        _lib.ptr(st.score_h), _lib.ptr(st.page_max), int(st.score_chunks),
-        _lib.ptr(st.n_pages), _lib.ptr(st.n_sel_hi), _lib.ptr(st.b_fix),
-        _lib.ptr(st.score), _lib.ptr(st.page_table), _lib.ptr(st.page_cnt),
-        _lib.ptr(st.sel_ws), st.sel_ws.numel(), int(n_req), int(st.n_kv), int(st.G),
+        st.score_h.data_ptr(), st.page_max.data_ptr(), int(st.score_chunks),
+        st.n_pages.data_ptr(), st.n_sel_hi.data_ptr(), st.b_fix.data_ptr(),
+        st.score.data_ptr(), st.page_table.data_ptr(), st.page_cnt.data_ptr(),
+        st.sel_ws.data_ptr(), st.sel_ws.numel(), int(n_req), int(st.n_kv), int(st.G),
         int(st.sink_pages), int(st.max_pages), combine, int(st.b_max),
         _lib.stream_ptr(st.score.device)),
         "select_nrm_topb")
