@@ -18,10 +18,14 @@ PPS_MIN_OVERRIDE = None        # set by bench sweeps; None = the table below
 
 
 def _pps_min(n_req: int) -> int:
-    """Minimum pages per split workgroup (the latent page is 18 KB)."""
+    """Minimum pages per split workgroup (the latent page is 18 KB): 4 at
+    every batch size.  A workgroup walks its pages one after the other, ~1.3 us
+    each, so more of them only lengthen it; two layers at 4 / 8 / 16 pages: 8
+    ragged requests 99 / 106 / 124 us, 16 x 16K 101 / 107 / 125, 24 x 8K
+    128 / 133, 32 x 4-8K 138 / 149 / 164 (12 pages)."""
     if PPS_MIN_OVERRIDE:
         return int(PPS_MIN_OVERRIDE)
-    return 4 if n_req <= 4 else 8
+    return 4
 
 
 def mla_decode(st, q, kv_cache, block_table, seq_lens, n_req: int, scale: float, out,
