@@ -693,6 +693,35 @@ __global__ __launch_bounds__(RF_THREADS) void refresh_compact_kernel(
     if (m) blocks[base + pre] = i;
 }
 
+// Tail mode for up to RF_THREADS rows in one launch: one workgroup takes each
+// row's last finalized page and lists the blocks that no earlier row has.  The
+// byte map is not needed (marking and compacting it took two launches for a
+// handful of rows: tail of 4 requests, 32 layers, 59.9 -> 56.9 us).
+__global__ __launch_bounds__(RF_THREADS) void refresh_tail_kernel(
+    const int* __restrict__ bt, long bt_sr, const int* __restrict__ sl, int n_req,
+    const int* __restrict__ rows, int n_rows, int page, int NB, int* __restrict__ blocks,
+    int* __restrict__ count)
+{
+    __shared__ int ids[RF_THREADS], n;
+    const int i = threadIdx.x;
+    int blk = -1;
+    if (i < n_rows) {
+        const int r = rows ? rows[i] : i;
+        if (r >= 0 && r < n_req) {
+            const int fin1 = min(max(sl[r] / page - 1, 0), (int)bt_sr - 1);   // last finalized page
+            blk = bt[(long)r * bt_sr + fin1];
+        }
+    }
+    ids[i] = blk;
+    if (i == 0) n = 0;
+    __syncthreads();
+    bool mine = blk >= 0 && blk < NB;
+    for (int j = 0; j < min(n_rows, i); ++j) mine = mine && ids[j] != blk;
+    if (mine) blocks[atomicAdd(&n, 1)] = blk;
+    __syncthreads();
+    if (i == 0) *count = n;
+}
+
 }  // namespace locks
 
 using namespace locks;
@@ -796,6 +825,11 @@ extern "C" int32_t locks_refresh_blocks(
                       "locks_refresh_blocks: delta needs k_layers, tag, n_layers, n_kv");
         LOCKS_REQUIRE(k_stride_tok % 8 == 0 && k_stride_block % 8 == 0 && k_stride_head % 8 == 0,
                       "locks_refresh_blocks: K strides must be multiples of 8 elements");
+    }
+    if (mode == LOCKS_REFRESH_TAIL && n_rows <= RF_THREADS) {
+        hipLaunchKernelGGL(refresh_tail_kernel, dim3(1), dim3(RF_THREADS), 0, (hipStream_t)stream, block_table,
+                           (long)bt_stride, seq_lens, n_req, rows, n_rows, page, num_blocks, blocks, count);
+        return check_launch("refresh_tail_kernel");
     }
     const long items = mode == LOCKS_REFRESH_TAIL ? (long)n_rows
                        : (long)n_req * max_fin * (mode == LOCKS_REFRESH_DELTA ? n_kv : 1);

@@ -768,8 +768,8 @@ __global__ __launch_bounds__(MH_BLK) void decode_merge_heads_kernel(
 // D / 64 columns of every split, all loaded at once; split weights sit one per
 // lane and are read by lane, so nothing goes through LDS and there is no
 // barrier.  Against the 256-thread form above, whose five barriers cost as
-// much as its loads: two layers of 16 requests 138.3 -> 135.2 us, of 4 ragged
-// 1M-class requests (three layers) 134.6 -> 133.7, one request within noise.
+// much as its loads: two layers of 16 requests 138.3 -> 135.2 us, of 4
+// requests of 64K to 256K tokens (three layers) 134.6 -> 133.7, one request within noise.
 // 32 splits: the most that the row count's pages-per-split rule launches at
 // the usual budgets, and what a lane's registers hold.
 template <int D, int NS>
