@@ -188,8 +188,12 @@ __device__ __forceinline__ float lanes_sum(float v) {
 //   4 layers x 512 pages x 8 heads, d 128 page 32    6.52 -> 0.96 ms
 //   4 layers x 256 pages x 8 heads, d 128 page 64    135 -> 3.85 ms
 //   32 layers x 8 heads x 4 pages (one a wave)       82 -> 60 us
-// Page 16 is now bound by VALU issue: 150 of a step's ~165 instructions are
-// VALU, four steps' worth of pages at once; the gram and the pack are 1/4.
+// What bounds page 16 now: the Jacobi takes 2/3 of the time, ~120 clocks per CU
+// for a wave's step of ~140-167 VALU instructions and 23 LDS operations (18
+// exchanges), four waves a SIMD.  Both pipes are near full: the schedule from a
+// table instead of arithmetic (27 VALU instructions fewer a step) gave 1 %, and
+// made a lone page slower (57 -> 61 us, its scalar loads wait).  The gram, the
+// pack and their loads are the rest.
 
 // Parallel cyclic Jacobi, round-robin ordering: index 0 stays, 1 .. N - 1
 // rotate.  At step s index i > 0 sits in slot 1 + (i - 1 - s) mod (N - 1);
