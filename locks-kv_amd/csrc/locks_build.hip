@@ -32,8 +32,9 @@ namespace locks {
 constexpr int BD_RNK = 8;
 // build grid cap (waves stride over the rest): a few resident rounds on 256 CUs
 constexpr long BD_MAX_GRID = 4096;
-// items up to which a wave builds one page instead of 64 / page: one wave per
-// SIMD of the chip (1024 pages: 60 us one a wave; 1600 to 4096: 70 us at four)
+// waves that the items are spread over before a wave takes another page (up to
+// 64 / page): one per SIMD of the chip.  1024 pages 60 us at one a wave; 1600
+// pages 63 us at two (70 at four), 2400 68 us at three (70), 4096 72 us at four
 constexpr long BD_SPREAD = 1024;
 
 // Per-wave LDS image of one page of locks_pack_rki4: PG tokens x D dims and
@@ -742,8 +743,8 @@ static int bd_launch(const uint16_t* kc, const uint64_t* k_layers, long k_sb, lo
                      int NB, const int* blocks, const int* count, int n_blocks, int n_kv,
                      int n_layers, long layer_rows, const SlabRows& S, uint16_t* tag, hipStream_t st) {
     const long items = (long)n_blocks * n_kv * n_layers;
-    // few items: one page per wave, on as many SIMDs as there are items
-    const int gpw = items <= BD_SPREAD ? 1 : kWave / PG;
+    // few items: fewer pages per wave, on as many SIMDs as there are items
+    const int gpw = (int)std::min<long>(kWave / PG, std::max<long>(1, (items + BD_SPREAD - 1) / BD_SPREAD));
     const long grid = std::min((items + 4 * gpw - 1) / (4 * gpw), BD_MAX_GRID);
     hipLaunchKernelGGL((rki4_build_kernel<D, PG>), dim3((unsigned)grid), dim3(4 * kWave), 0, st, kc,
                        k_layers, k_sb, k_st, k_sh, NB, blocks, count, n_blocks, n_kv, n_layers,
