@@ -305,10 +305,14 @@ __device__ __forceinline__ void jacobi(float (&A)[N], float (&U)[N], float& diag
 }
 
 // a / b, correctly rounded, from y = RN(1 / b): the quotient estimate a y and
-// one residual correction (Markstein 1990; exact away from under- / overflow).
+// one residual correction (Markstein 1990; exact away from under- / overflow:
+// scales are at least 1e-8, so what underflows is a zero code either way).
+// b infinite (a page with infinite keys, or an overflowing gram): y is 0 and
+// the residual is taken against 0 in place of b, so a finite a gives 0 and
+// not NaN.  The select is one per scale, not per quotient.
 __device__ __forceinline__ float div_by(float a, float b, float y) {
-    const float q = a * y;
-    return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+    const float q = a * y, br = y == 0.f ? 0.f : b;
+    return __builtin_fmaf(__builtin_fmaf(-q, br, a), y, q);
 }
 
 typedef const __attribute__((address_space(1))) uint32_t* global_u32;
