@@ -82,7 +82,8 @@ def slab_row_bytes(slabs) -> "ctypes.Array":
     vals = []
     for t, tail in zip(slabs, (2, 1, 2, 1, 1, 0)):    # field dims after (NB, n_kv)
         kv_dim = t.dim() - tail - 1
-        rb = t.stride(kv_dim) * t.element_size()
+        # (one kv head: torch gives a dim of size 1 any stride, the block's counts)
+        rb = t.stride(kv_dim if t.shape[kv_dim] > 1 else kv_dim - 1) * t.element_size()
         assert t.stride(kv_dim - 1) * t.element_size() == rb * t.shape[kv_dim], \
             "slab rows of one block must be consecutive over kv heads"
         vals.append(rb)
