@@ -111,12 +111,20 @@ __global__ __launch_bounds__(SC_BLOCK) void rki4_score_kernel(
     constexpr int LPH = D / QDL;            // q lanes per head (8 or 16: one DPP row group)
     const int h = blockIdx.y, r = blockIdx.z;                   // kv head, request
     const int Z = gridDim.x;
-    // Page chunk, rotated by the request: workgroups go round the 8 XCDs in
-    // grid order, so with Z x n_kv a multiple of 8 chunk z of every request
-    // would land on one XCD, and the last chunks exist in long requests only
-    // (16 requests of 3K to 32K tokens, Z = 8: scorer 35.5 -> 28.1 us, the
-    // step's layer 76 -> 70 us; uniform and one-request grids unchanged).
-    const int z = (int)((blockIdx.x + (unsigned)r) % (unsigned)Z);
+    // Page chunk, rotated by the request inside groups of Z's largest power of
+    // two.  Workgroups go round the 8 XCDs, and an XCD's round its shader
+    // engines, in grid order: where Z x n_kv shares that power of two with
+    // them, chunk z of every request would land on the same ones, and the last
+    // chunks exist in long requests only (16 requests of 3K to 32K tokens,
+    // Z = 8: scorer 34.1 -> 25.1 us; G = 16, Z = 32: 14.5 -> 11.3).  An odd Z
+    // moves the chunks by itself.  (Rotating any Z by a modulo cost its ~40
+    // scalar instructions before the first load and moved grids that needed
+    // nothing: Z = 22, 3 ragged requests 5.3 -> 6.1 us, 4 uniform requests at
+    // Z = 32 13.4 -> 14.0; so rotated 5.3 and 13.4.  By XOR, requests sorted by
+    // length keep their longest chunks together: 16 heads, 8 requests 36.8 ->
+    // 37.3 instead of 28.0.)
+    const int zm = (Z & -Z) - 1;
+    const int z = ((int)blockIdx.x & ~zm) | (((int)blockIdx.x + r) & zm);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int P = min(nsh[r], MP);          // never score past the score_h row
     const int c0 = z * chunk;
