@@ -505,23 +505,27 @@ constexpr int ROW_NW = ROW_BLK / kWave;
 // 20.5 us; G = 16: 44.8 vs 25.7 us).
 constexpr int ROW_MAXP = 8 * ROW_BLK;
 
-// Rows of score_h and page_table start 4-byte aligned when max_pages is not a
-// multiple of 4: vector accesses of that alignment.
-typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
+// An odd row of the chunk kernel starts 4-byte aligned.
 typedef float f2a4 __attribute__((ext_vector_type(2), aligned(4)));
-typedef int i4a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// ROW: the row's length -- 0: a multiple of 4 pages; 1: any other of at least
-// 4; 2: at most 3.  (As run-time branches around the loads the other two made
-// every load wait at a join: step 129 -> 142 us at 128K.)
-template <int E, int HB, int ROW>
+// ODD: the row's length is not a multiple of 4, so rows start 4-byte aligned.
+// A misaligned 16-byte load costs about a clock per lane, whatever the row's
+// length (16 heads x 16 waves of them ~7 us), so an odd row is combined from
+// coalesced dwords -- thread t takes pages t, t + 1024, .. -- and the sums
+// change hands through LDS for the selection; a row of at most 1024 pages
+// (E = 1) needs neither.  16-byte loads against dwords, G = 16, 64 requests,
+// 63 pages kept whole / 126 of 1023: 13.2 / 16.1 -> 4.1 / 6.3 us (rows of 64 /
+// 1024 pages: 6.2 / 9.2); G = 4, one request, 5001 pages: 11.1 -> 8.6.  (A
+// template: as run-time branches around the loads the forms made every load
+// wait at a join, step 129 -> 142 us at 128K.)
+template <int E, int HB, bool ODD>
 __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     const float* __restrict__ score_h, const float* __restrict__ pmax, int Zs,
     const int* __restrict__ npg, const int* __restrict__ nsh, const int* __restrict__ bfix,
     float* __restrict__ score, int* __restrict__ page_table, int* __restrict__ page_cnt,
     int n_sink, int MP, int G, int combine)
 {
-    static_assert(E % 4 == 0, "pages per thread must be a multiple of 4");
+    static_assert(E % 4 == 0 || (ODD && E == 1), "pages per thread: a multiple of 4, or 1");
     const int kh = blockIdx.x, r = blockIdx.y, n_kv = gridDim.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const long rk = (long)r * n_kv + kh;
@@ -532,10 +536,12 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     int b = bfix[r];
     b = max(1, min(b, max(n_sel, 1)));
     const int pend = max(n_sel_hi, 0);                    // score written for p < pend
-    const int p0 = tid * E;
+    const int p0 = tid * E;                               // this thread's pages in the selection
+    auto load_page = [&](int e) { return ODD ? tid + ROW_BLK * e : p0 + e; };   // and in the combine
 
     __shared__ float hm[16];
     __shared__ int hist[4096];
+    __shared__ __attribute__((aligned(16))) float turn[ODD && E > 1 ? ROW_BLK * E : 4];
     __shared__ int wtot[ROW_NW];
     __shared__ int s3[4];
     __shared__ int wsum[ROW_NW + 1];
@@ -552,35 +558,25 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     // HB heads per load batch: the host passes 4 for groups of at most 4
     // (the clamped loads of heads past G re-read the last head)
     const float* shb = score_h + rk * (long)G * MP;
-    float4 xv[HB][E / 4];
+    float xv[HB][E];
     auto load_batch = [&](int g0) {
 #pragma unroll
-        for (int j = 0; j < HB; ++j)
+        for (int j = 0; j < HB; ++j) {
+            // unconditional (clamped) loads: surplus heads / pages are
+            // never combined or kept, and a guarded load would make the
+            // compiler wait for it before the page maxima are requested
+            const float* row = shb + (long)min(g0 + j, G - 1) * MP;
+            if constexpr (ODD) {
 #pragma unroll
-            for (int v = 0; v < E / 4; ++v) {
-                // unconditional (clamped) loads: surplus heads / pages are
-                // never combined or kept, and a guarded load would make the
-                // compiler wait for it before the page maxima are requested
-                const float* row = shb + (long)min(g0 + j, G - 1) * MP;
-                const int p = p0 + 4 * v;
-                if constexpr (ROW == 0) {
-                    xv[j][v] = *reinterpret_cast<const float4*>(row + min(p, MP - 4));
-                } else if constexpr (ROW == 1) {
-                    const f4a4 x = *reinterpret_cast<const f4a4*>(row + min(p, MP - 4));
-                    xv[j][v] = make_float4(x[0], x[1], x[2], x[3]);
-                } else {
-                    xv[j][v] = make_float4(row[min(p, MP - 1)], row[min(p + 1, MP - 1)], row[min(p + 2, MP - 1)],
-                                           row[MP - 1]);
+                for (int e = 0; e < E; ++e) xv[j][e] = row[min(load_page(e), MP - 1)];
+            } else {
+#pragma unroll
+                for (int v = 0; v < E / 4; ++v) {
+                    const float4 x = *reinterpret_cast<const float4*>(row + min(p0 + 4 * v, MP - 4));
+                    xv[j][4 * v] = x.x; xv[j][4 * v + 1] = x.y; xv[j][4 * v + 2] = x.z; xv[j][4 * v + 3] = x.w;
                 }
             }
-    };
-    // A row of 4 k + 1 .. 3 pages: the one thread whose vector runs past it
-    // loaded the row's last four and takes its pages from the vector's end.
-    auto tail_shift = [&](float (&x)[4], int p) {
-        const int sh = p < MP ? p - (MP - 4) : 0;
-        x[0] = sh == 1 ? x[1] : sh == 2 ? x[2] : sh == 3 ? x[3] : x[0];
-        x[1] = sh == 1 ? x[2] : sh >= 2 ? x[3] : x[1];
-        x[2] = sh >= 1 ? x[3] : x[2];
+        }
     };
     load_batch(0);
     if (combine == 0) {
@@ -605,14 +601,9 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
                 const bool on = g0 + j < G;
                 const float h = hm[min(g0 + j, G - 1)];
 #pragma unroll
-                for (int v = 0; v < E / 4; ++v) {
-                    float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
-                    if constexpr (ROW == 1) tail_shift(x4, p0 + 4 * v);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float t = __expf(x4[i] - h);
-                        acc[4 * v + i] = on ? acc[4 * v + i] + t : acc[4 * v + i];
-                    }
+                for (int e = 0; e < E; ++e) {
+                    const float t = __expf(xv[j][e] - h);
+                    acc[e] = on ? acc[e] + t : acc[e];
                 }
             }
         } else {
@@ -620,34 +611,29 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
             for (int j = 0; j < HB; ++j) {
                 const int g = g0 + j;
 #pragma unroll
-                for (int v = 0; v < E / 4; ++v) {
-                    float x4[4] = {xv[j][v].x, xv[j][v].y, xv[j][v].z, xv[j][v].w};
-                    if constexpr (ROW == 1) tail_shift(x4, p0 + 4 * v);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float mx = (g == 0) ? x4[i] : fmaxf(acc[4 * v + i], x4[i]);
-                        acc[4 * v + i] = (g < G) ? mx : acc[4 * v + i];
-                    }
+                for (int e = 0; e < E; ++e) {
+                    const float mx = (g == 0) ? xv[j][e] : fmaxf(acc[e], xv[j][e]);
+                    acc[e] = (g < G) ? mx : acc[e];
                 }
             }
         }
     }
     float* srow = score + rk * (long)MP;
-    if (p0 + E <= pend) {
+    if (!ODD && p0 + E <= pend) {
 #pragma unroll
         for (int v = 0; v < E / 4; ++v)
-            *reinterpret_cast<f4a4*>(srow + p0 + 4 * v) = f4a4{acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]};
+            *reinterpret_cast<float4*>(srow + p0 + 4 * v) = make_float4(acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]);
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (p0 + e < pend) srow[p0 + e] = acc[e];
+            if (load_page(e) < pend) srow[load_page(e)] = acc[e];
     }
 
     int* trow = page_table + rk * (long)MP;
     if (keep_all || b >= n_sel) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int i = p0 + e;
+            const int i = load_page(e);
             if (i < MP) trow[i] = (i < n_pages) ? i : -1;
         }
         if (tid == 0) page_cnt[rk] = n_pages;
@@ -658,13 +644,13 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     // padding -- are stored before the select, so their stores drain under
     // it instead of ahead of the kernel's end (Llama 128K row: -0.5 us)
     const int cnt = n_sink + b + (n_pages - n_sel_hi);
-    if (p0 >= cnt && p0 + E <= MP) {                      // padding only
+    if (!ODD && p0 >= cnt && p0 + E <= MP) {              // padding only
 #pragma unroll
-        for (int v = 0; v < E / 4; ++v) *reinterpret_cast<i4a4*>(trow + p0 + 4 * v) = i4a4{-1, -1, -1, -1};
-    } else if (p0 < n_sink || p0 + E > n_sink + b) {     // not only kept slots
+        for (int v = 0; v < E / 4; ++v) *reinterpret_cast<int4*>(trow + p0 + 4 * v) = make_int4(-1, -1, -1, -1);
+    } else if (ODD || p0 < n_sink || p0 + E > n_sink + b) {   // not only kept slots
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int i = p0 + e;
+            const int i = load_page(e);
             if (i >= MP) break;
             if (i < n_sink) trow[i] = i;
             else if (i >= n_sink + b && i < cnt) trow[i] = n_sel_hi + (i - n_sink - b);
@@ -674,6 +660,16 @@ __global__ __launch_bounds__(ROW_BLK) void sel_row_kernel(
     if (tid == 0) page_cnt[rk] = cnt;
 
     // ---- exact b-th largest key among the selectable pages [n_sink, nsh) --
+    if constexpr (ODD && E > 1) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) turn[load_page(e)] = acc[e];
+        lds_barrier();
+#pragma unroll
+        for (int v = 0; v < E / 4; ++v) {
+            const float4 x = *reinterpret_cast<const float4*>(&turn[p0 + 4 * v]);
+            acc[4 * v] = x.x; acc[4 * v + 1] = x.y; acc[4 * v + 2] = x.z; acc[4 * v + 3] = x.w;
+        }
+    }
     uint32_t key[E];
     bool val[E];
 #pragma unroll
@@ -1147,13 +1143,8 @@ extern "C" int32_t locks_select_nrm_topb(
 #ifndef SEL_ROW_MAX_GP
 #define SEL_ROW_MAX_GP 65536L
 #endif
-    // The row kernel also serves rows of one chunk or less: against the
-    // single-chunk kernel it measured GLM 16K 1.225 -> 1.083 ms and 32K
-    // 1.327 -> 1.104 ms per step
-    // Both routes take rows of any length.  A page count that is not a multiple
-    // of 4 took a 512-thread chunk kernel and, past 2048 pages, a second launch:
-    // step of two layers at 50001 tokens 93 -> 57 us, 20001 65 -> 52, 300001
-    // 132 -> 99 (10 % budget 246 -> 162), G = 16 at 150100 104 -> 69.
+    // Both routes take rows of any length, and the row kernel also rows of one
+    // chunk or less (one launch in place of two).
     if (max_pages <= ROW_MAXP && (long)G * max_pages <= SEL_ROW_MAX_GP) {
 #define ROW_LAUNCH(EV, HBV, RV)                                                                \
         hipLaunchKernelGGL((sel_row_kernel<EV, HBV, RV>), dim3(n_kv, n_req), dim3(ROW_BLK), 0, st, score_h, \
@@ -1167,14 +1158,13 @@ extern "C" int32_t locks_select_nrm_topb(
             else if (G <= 4) ROW_LAUNCH(EV, 4, RV);                                            \
             else ROW_LAUNCH(EV, 8, RV);                                                        \
         } while (0)
-        if (max_pages < 4) ROW_LAUNCH(4, 8, 2);
-        else if (max_pages <= 4 * ROW_BLK) {
-            if (max_pages % 4 == 0) ROW_LAUNCH_G(4, 0);
-            else ROW_LAUNCH_G(4, 1);
-        } else {
-            if (max_pages % 4 == 0) ROW_LAUNCH_G(8, 0);
-            else ROW_LAUNCH_G(8, 1);
-        }
+        // odd rows of at most 1024 pages: a page per thread
+        if (max_pages % 4 == 0) {
+            if (max_pages <= 4 * ROW_BLK) ROW_LAUNCH_G(4, false);
+            else ROW_LAUNCH_G(8, false);
+        } else if (max_pages <= ROW_BLK) ROW_LAUNCH_G(1, true);
+        else if (max_pages <= 4 * ROW_BLK) ROW_LAUNCH_G(4, true);
+        else ROW_LAUNCH_G(8, true);
 #undef ROW_LAUNCH_G
 #undef ROW_LAUNCH
         return check_launch("sel_row_kernel");
