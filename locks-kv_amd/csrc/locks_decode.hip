@@ -768,10 +768,9 @@ __global__ __launch_bounds__(MH_BLK) void decode_merge_heads_kernel(
 // D / 64 columns of every split, all loaded at once; split weights sit one per
 // lane and are read by lane, so nothing goes through LDS and there is no
 // barrier.  Against the 256-thread form above, whose five barriers cost as
-// much as its loads: two layers of 16 requests 138.3 -> 135.2 us, of 4
-// requests of 64K to 256K tokens (three layers) 134.6 -> 133.7, one request within noise.
-// 32 splits: the most that the row count's pages-per-split rule launches at
-// the usual budgets, and what a lane's registers hold.
+// much as its loads: up to 16 splits 3.2-3.5 -> 2.4-2.9 us for one request at
+// any D, 8.8 -> 4.2-5.2 for 4096 heads (two layers of 16 requests 138.3 ->
+// 135.2 us).  17 to 32 splits: merge_wave32_heads.
 template <int D, int NS>
 __global__ __launch_bounds__(kWave) void decode_merge_wave_kernel(
     const float* __restrict__ m_part, const float* __restrict__ l_part,
@@ -815,6 +814,15 @@ __global__ __launch_bounds__(kWave) void decode_merge_wave_kernel(
         for (int c = 0; c < CPL; ++c) static_cast<uint16_t*>(out)[oi + c] = f32_to_bf16(acc[c] * inv);
     }
 }
+
+// Heads past which the one-wave form is the faster one at 17 to 32 splits of
+// d 256: one wave issues all their loads, 32 x D / 64 registers of them, and a
+// head of 1 KB a split needs many waves in flight to hide that.  256-thread
+// form / one wave, 32 splits: 3.2 / 3.7 us at 32 heads, 5.3 / 5.3 at 1024, 14.5 /
+// 13.3 at 2048 (four layers, one request, G = 16: step 124.5 / 125.4 us).  At d 64
+// and 128 the wave is never slower in a step (d 128, 17 to 32 splits: four layers
+// 101.6 / 100.7 to 104.2 / 103.3 us).
+constexpr long merge_wave32_heads(int d) { return d <= 128 ? 0 : 1792; }
 
 // ---- no-allocation variant of the fused decode ----------------------------
 // Scratch of locks_decode_fused_noalloc: the arrival counters (first 256-B
@@ -1040,6 +1048,7 @@ extern "C" int32_t locks_decode_merge(
                   "locks_decode_merge: out strides must be multiples of 4 elements");
     if (n_req == 0) return 0;
     const int nsplit = launched_splits(split, pps_min, max_cnt);
+    const long heads = (long)n_req * n_kv * G;
     hipStream_t st = (hipStream_t)stream;
 #define LAUNCH_WAVE(DV, NSV)                                                                        \
     hipLaunchKernelGGL((decode_merge_wave_kernel<DV, NSV>), dim3(G, n_kv, n_req), dim3(kWave), 0, st, \
@@ -1048,7 +1057,7 @@ extern "C" int32_t locks_decode_merge(
 #define LAUNCH_D(DV)                                                                                \
     if (nsplit <= 8) LAUNCH_WAVE(DV, 8);                                                            \
     else if (nsplit <= 16) LAUNCH_WAVE(DV, 16);                                                     \
-    else if (nsplit <= 32) LAUNCH_WAVE(DV, 32);                                                     \
+    else if (nsplit <= 32 && heads > merge_wave32_heads(DV)) LAUNCH_WAVE(DV, 32);                   \
     else hipLaunchKernelGGL(decode_merge_heads_kernel<DV>, dim3(G, n_kv, n_req), dim3(MH_BLK), 0,   \
                        st, m_part, l_part, acc_part, page_cnt, (long)cnt_stride,                    \
                        pt_cols, nullptr, 1, out, (long)out_stride_req, (long)out_stride_head,       \
