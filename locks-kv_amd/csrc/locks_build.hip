@@ -703,15 +703,24 @@ __global__ __launch_bounds__(RF_THREADS) void refresh_compact_kernel(
 }
 
 // Tail mode for up to RF_THREADS rows in one launch: one workgroup takes each
-// row's last finalized page and lists the blocks that no earlier row has.  The
-// byte map is not needed (marking and compacting it took two launches for a
-// handful of rows: tail of 4 requests, 32 layers, 59.9 -> 56.9 us).
+// row's last finalized page and lists each block once.  The byte map is not
+// needed (marking and compacting it took two launches for a handful of rows:
+// tail of 4 requests, 32 layers, 59.9 -> 56.9 us).  Duplicates collapse in an
+// LDS hash table, whose time does not grow with the rows: two launches 3.7 / 4.4 /
+// 6.5 us at 4 / 64 / 256 rows, this one 2.1 / 2.1 / 2.3 (with each row compared to
+// all earlier ones 2.2 / 5.2 / 14.8).  Two multiplications spread blocks at any
+// regular distance (a table's width): 256 of them probe 17 slots at worst for
+// distances up to 4200 (one multiplication: 256).  There are at most RF_THREADS
+// blocks in RF_SLOTS slots, so a probe ends at its block or at a free slot.
+constexpr int RF_SLOT_BITS = 10, RF_SLOTS = 1 << RF_SLOT_BITS;
+static_assert(RF_SLOTS == 4 * RF_THREADS, "four slots a thread");
 __global__ __launch_bounds__(RF_THREADS) void refresh_tail_kernel(
     const int* __restrict__ bt, long bt_sr, const int* __restrict__ sl, int n_req,
     const int* __restrict__ rows, int n_rows, int page, int NB, int* __restrict__ blocks,
     int* __restrict__ count)
 {
-    __shared__ int ids[RF_THREADS], n;
+    __shared__ __attribute__((aligned(16))) int slot[RF_SLOTS];
+    __shared__ int n;
     const int i = threadIdx.x;
     int blk = -1;
     if (i < n_rows) {
@@ -721,12 +730,18 @@ __global__ __launch_bounds__(RF_THREADS) void refresh_tail_kernel(
             blk = bt[(long)r * bt_sr + fin1];
         }
     }
-    ids[i] = blk;
+    *reinterpret_cast<int4*>(&slot[4 * i]) = make_int4(-1, -1, -1, -1);
     if (i == 0) n = 0;
     __syncthreads();
-    bool mine = blk >= 0 && blk < NB;
-    for (int j = 0; j < min(n_rows, i); ++j) mine = mine && ids[j] != blk;
-    if (mine) blocks[atomicAdd(&n, 1)] = blk;
+    if (blk >= 0 && blk < NB) {
+        uint32_t h = (uint32_t)blk * 0x9E3779B1u;
+        h = (h ^ (h >> 15)) * 0x85EBCA77u;
+        for (int at = (int)(h >> (32 - RF_SLOT_BITS));; at = (at + 1) & (RF_SLOTS - 1)) {
+            const int had = atomicCAS(&slot[at], -1, blk);
+            if (had == -1) blocks[atomicAdd(&n, 1)] = blk;           // this row is the first with the block
+            if (had == -1 || had == blk) break;
+        }
+    }
     __syncthreads();
     if (i == 0) *count = n;
 }
