@@ -36,6 +36,16 @@ constexpr long BD_MAX_GRID = 4096;
 // 64 / page): one per SIMD of the chip.  1024 pages 60 us at one a wave; 1600
 // pages 63 us at two (70 at four), 2400 68 us at three (70), 4096 72 us at four
 constexpr long BD_SPREAD = 1024;
+// pages per wave, at most gw (1, 2 or 4), of `items` on `waves` waves.  The host
+// sizes the grid with it for the bound that it knows; the kernel packs what the
+// device count says (8 layers, 4 blocks to build of a bound of 2048, packed by
+// the bound / by the count: d 512 89 / 58 us, 8 heads of d 128 58 / 49).
+__host__ __device__ __forceinline__ int pages_per_wave(long items, long waves, int gw) {
+    const long n = waves < BD_SPREAD ? waves : BD_SPREAD;
+    int g = 1;
+    for (int k = 1; k < gw; ++k) g += items > k * n ? 1 : 0;
+    return g;
+}
 
 // Per-wave LDS image of one page of locks_pack_rki4: PG tokens x D dims and
 // the caller's eigenvectors.
@@ -336,8 +346,8 @@ struct BuildLds {
     };
 };
 
-// Grid: one wave per gpw (1 to 64 / PG) consecutive (layer, block, kv head)
-// items, waves stride over the rest.  Layer l reads K from k_layers[l] (or kc
+// One wave takes gpw (1 to 64 / PG) consecutive (layer, block, kv head) items at a
+// time, and waves stride over the rest.  Layer l reads K from k_layers[l] (or kc
 // for a single-layer call) and writes slab rows offset by l * layer_rows.
 // n_dev, when given, is a device count of valid entries of `blocks` (at most
 // n_blocks): the refresh producers size the grid to the host-known bound and
@@ -347,7 +357,7 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
     const uint16_t* __restrict__ kc, const uint64_t* __restrict__ k_layers,
     long k_sb, long k_st, long k_sh, int NB,
     const int* __restrict__ blocks, const int* __restrict__ n_dev, int n_blocks, int n_kv,
-    int n_layers, long layer_rows, SlabRows S, uint16_t* __restrict__ tag, int gpw)
+    int n_layers, long layer_rows, SlabRows S, uint16_t* __restrict__ tag)
 {
     using LDS = BuildLds<PG>;
     constexpr int NW = 4, GW = LDS::GW, NB16 = PG / 16;
@@ -359,6 +369,7 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
     LDS& L = lds[wave];
     const int nb_valid = n_dev ? min(*n_dev, n_blocks) : n_blocks;
     const long per_layer = (long)nb_valid * n_kv, total = per_layer * n_layers;
+    const int gpw = pages_per_wave(total, (long)gridDim.x * NW, GW);
     const int j = lane & (PG - 1), pg = lane / PG;   // this lane's column / token, and page
     const bool own = lane < LPP;                     // d = 64: the upper lanes repeat, and store nothing
     const int cl = own ? lane : lane - LPP;
@@ -762,12 +773,11 @@ static int bd_launch(const uint16_t* kc, const uint64_t* k_layers, long k_sb, lo
                      int NB, const int* blocks, const int* count, int n_blocks, int n_kv,
                      int n_layers, long layer_rows, const SlabRows& S, uint16_t* tag, hipStream_t st) {
     const long items = (long)n_blocks * n_kv * n_layers;
-    // few items: fewer pages per wave, on as many SIMDs as there are items
-    const int gpw = (int)std::min<long>(kWave / PG, std::max<long>(1, (items + BD_SPREAD - 1) / BD_SPREAD));
+    const int gpw = pages_per_wave(items, BD_SPREAD, kWave / PG);
     const long grid = std::min((items + 4 * gpw - 1) / (4 * gpw), BD_MAX_GRID);
     hipLaunchKernelGGL((rki4_build_kernel<D, PG>), dim3((unsigned)grid), dim3(4 * kWave), 0, st, kc,
                        k_layers, k_sb, k_st, k_sh, NB, blocks, count, n_blocks, n_kv, n_layers,
-                       layer_rows, S, tag, gpw);
+                       layer_rows, S, tag);
     return check_launch("rki4_build_kernel");
 }
 #define BD_DISPATCH(HD, PGV, ...)                                              \

@@ -1,7 +1,7 @@
-"""The builder packs 64 / page pages into a wave once there are more items than
-SIMDs to spread them over: every packing (full waves, partial last waves, masked
-block ids among them) writes the bytes that a page built alone gets, and
-leaves every other record untouched.  A page's build depends on that page
+"""The builder packs up to 64 / page pages into a wave once there are more items
+than SIMDs to spread them over: one and two pages a wave (full waves, partial
+last waves, masked block ids among them) write the bytes that a page built alone gets, and
+leave every other record untouched.  A page's build depends on that page
 alone and takes the same roundings in any packing, so the bytes are equal."""
 import numpy as np
 import pytest
@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 SLABS = ("pp_v4", "pp_vs", "pp_c8", "pp_cs", "pp_mu8", "pp_mus", "pp_tag")
 
 
-# items per call: below, at and above the spread limit (1024), odd remainders
-# of 2, 4 and 16 pages per wave
+# items per call: below, at and just above the spread limit (1024), with odd
+# remainders of two pages a wave (page 64: always one)
 @pytest.mark.parametrize("d,page,n_kv,n_blocks", [
     (128, 16, 2, 1), (128, 16, 8, 128), (128, 16, 5, 205), (128, 16, 3, 343), (64, 16, 2, 515),
     (256, 16, 2, 513), (512, 16, 1, 1027), (128, 32, 2, 513), (64, 64, 2, 514), (256, 64, 3, 343)])
