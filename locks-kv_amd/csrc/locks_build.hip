@@ -318,10 +318,11 @@ __device__ __forceinline__ void jacobi(float (&A)[N], float (&U)[N], float& diag
 // one residual correction (Markstein 1990; exact away from under- / overflow:
 // scales are at least 1e-8, so what underflows is a zero code either way).
 // b infinite (a page with infinite keys, or an overflowing gram): y is 0 and
-// the residual is taken against 0 in place of b, so a finite a gives 0 and
-// not NaN.  The select is one per scale, not per quotient.
-__device__ __forceinline__ float div_by(float a, float b, float y) {
-    const float q = a * y, br = y == 0.f ? 0.f : b;
+// the residual is taken against br = 0 in place of b, so a finite a gives 0
+// and not NaN.
+__device__ __forceinline__ float residual_divisor(float b, float y) { return y == 0.f ? 0.f : b; }
+__device__ __forceinline__ float div_by(float a, float br, float y) {
+    const float q = a * y;
     return __builtin_fmaf(__builtin_fmaf(-q, br, a), y, q);
 }
 
@@ -340,7 +341,7 @@ struct BuildLds {
         float2 cs[GW][PG / 2];
         struct {
             float u[GW][BD_RNK][PG];
-            float s8[GW][BD_RNK], y8[GW][BD_RNK];
+            float s8[GW][BD_RNK], r8[GW][BD_RNK], y8[GW][BD_RNK];    // values, residual divisors, reciprocals
             uint32_t lam[kWave];
         } top;
     };
@@ -493,8 +494,10 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
             if (rank >= PG - BD_RNK) {
                 const int r = rank - (PG - BD_RNK);
                 const float s8 = __fsqrt_rn(fmaxf(diag, 1e-10f));
+                const float y8 = __fdiv_rn(1.f, s8);
                 L.top.s8[pg][r] = s8;
-                L.top.y8[pg][r] = __fdiv_rn(1.f, s8);
+                L.top.r8[pg][r] = residual_divisor(s8, y8);
+                L.top.y8[pg][r] = y8;
             }
             L.top.lam[lane] = (uint32_t)rank;        // (every key has been read)
             wave_lds_sync();
@@ -517,11 +520,11 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
                     C[r] = __fmul_rn(L.top.u[pg][r][j], L.top.s8[pg][r]);
                     am = fmaxf(am, fabsf(C[r]));
                 }
-                const float csc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f), y = __fdiv_rn(1.f, csc);
+                const float csc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f), y = __fdiv_rn(1.f, csc), cr = residual_divisor(csc, y);
                 uint32_t wd[2] = {0u, 0u};
 #pragma unroll
                 for (int r = 0; r < BD_RNK; ++r) {
-                    const int q = (int)fminf(fmaxf(rintf(div_by(C[r], csc, y)), -127.f), 127.f);
+                    const int q = (int)fminf(fmaxf(rintf(div_by(C[r], cr, y)), -127.f), 127.f);
                     wd[r >> 2] |= (uint32_t)(q & 255) << (8 * (r & 3));
                 }
                 *reinterpret_cast<uint2*>(S.c8 + rwl * S.sc8 + j * BD_RNK) = make_uint2(wd[0], wd[1]);
@@ -549,9 +552,9 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
                         a = __fadd_rn(a, __fmul_rn(x[t][0], u));
                         b = __fadd_rn(b, __fmul_rn(x[t][1], u));
                     }
-                    const float s8 = L.top.s8[g][r], y8 = L.top.y8[g][r];
-                    V[k][0][r] = div_by(a, s8, y8);
-                    V[k][1][r] = div_by(b, s8, y8);
+                    const float r8 = L.top.r8[g][r], y8 = L.top.y8[g][r];
+                    V[k][0][r] = div_by(a, r8, y8);
+                    V[k][1][r] = div_by(b, r8, y8);
                 }
             }
             // Maxima over the channels of the 8 columns and the centroid.  Two
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
             }
             const float am = i16 == 0 ? m[0] : i16 == 1 ? m[1] : mm;
             const float sc = fmaxf(__fdiv_rn(am, i16 < 2 ? 7.f : 127.f), 1e-8f);
-            const float ys = __fdiv_rn(1.f, sc);
+            const float ys = __fdiv_rn(1.f, sc), sr = residual_divisor(sc, ys);
             if (i16 < 2)
                 reinterpret_cast<uint16_t*>(S.vs + rw * S.svs)[4 * i16 + 2 * (kq & 1) + (kq >> 1)] = f32_to_bf16(sc);
             if (lane == 2) *reinterpret_cast<uint16_t*>(S.mus + rw * S.smus) = f32_to_bf16(sc);
@@ -594,7 +597,7 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
 #pragma unroll
             for (int r = 0; r < BD_RNK; ++r) {
                 const int at = 16 * (((r & 1) << 1) | ((r >> 1) & 1)) + (r >> 2);   // the lane of column r
-                const float b = of_lane(sc, at), y = of_lane(ys, at);
+                const float b = of_lane(sr, at), y = of_lane(ys, at);
 #pragma unroll
                 for (int k = 0; k < NK; ++k) {
                     const int lo = (int)fminf(fmaxf(rintf(div_by(V[k][0][r], b, y)), -8.f), 7.f);
@@ -602,7 +605,7 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
                     if (own) vrow[r * (D / 2) + 64 * k + lane] = (uint8_t)((lo & 15) | ((hi & 15) << 4));
                 }
             }
-            const float b = of_lane(sc, 2), y = of_lane(ys, 2);
+            const float b = of_lane(sr, 2), y = of_lane(ys, 2);
 #pragma unroll
             for (int k = 0; k < NK; ++k) {
                 const int lo = (int)fminf(fmaxf(rintf(div_by(mu[k][0], b, y)), -127.f), 127.f);
