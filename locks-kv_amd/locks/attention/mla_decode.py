@@ -14,18 +14,34 @@ import torch
 from .. import _lib
 
 
-PPS_MIN_OVERRIDE = None        # set by bench sweeps; None = the table below
+PPS_MIN_OVERRIDE = None        # set by bench sweeps; None = the rule below
 
 
-def _pps_min(n_req: int) -> int:
-    """Minimum pages per split workgroup (the latent page is 18 KB): 4 at
-    every batch size.  A workgroup walks its pages one after the other, ~1.3 us
-    each, so more of them only lengthen it; two layers at 4 / 8 / 16 pages: 8
-    ragged requests 99 / 106 / 124 us, 16 x 16K 101 / 107 / 125, 24 x 8K
-    128 / 133, 32 x 4-8K 138 / 149 / 164 (12 pages)."""
+def _pps_min(n_req: int, max_cnt: int) -> int:
+    """Minimum pages per split workgroup (the latent page is 18 KB) of rows of
+    at most max_cnt pages: 4 while that makes at most two workgroups per CU
+    (512), else 8.  A workgroup walks its pages one after the other, ~1.3 us
+    each, so more of them lengthen it as long as CUs are idle; past that the
+    partials (32 KB a split, written and read again) and further rounds of
+    workgroups cost more.  Split + merge at 4 / 8 pages, 128 attended: 8 requests
+    17.9 / 20.6 us, 16 (512 workgroups) 21.8 / 21.1, 20 26.9 / 25.5, 32 37.8 /
+    28.2, 128 120 / 93; 200 attended: 10 requests 22.0 / 21.0, 12 26.7 / 25.2, 128
+    185 / 141; 100 attended: 20 requests 21.8 / 24.3, 24 26.4 / 25.1."""
     if PPS_MIN_OVERRIDE:
         return int(PPS_MIN_OVERRIDE)
-    return 4
+    return 4 if int(n_req) * -(-int(max_cnt) // 4) <= 512 else 8
+
+
+def _launch_shape(st, n_req: int):
+    """(pages per split, splits launched): the splits that a row under the
+    state's budget can fill.  Workgroups of splits past a row's end return at
+    once, but the dispatcher deals them out like the others: with 8 of 16 a row
+    empty, whole shader engines got nothing but those (32 requests at 8 pages,
+    128 attended: 45.0 -> 28.2 us with 16 of 32 splits launched).  A longer row
+    takes more pages per split."""
+    max_cnt = int(st.budget_abs) + int(st.sink_pages) + int(st.window_pages)
+    pps = _pps_min(n_req, max_cnt)
+    return pps, min(int(st.split), -(-max_cnt // pps))
 
 
 def mla_decode(st, q, kv_cache, block_table, seq_lens, n_req: int, scale: float, out,
@@ -40,7 +56,7 @@ def mla_decode(st, q, kv_cache, block_table, seq_lens, n_req: int, scale: float,
         raise TypeError("lse must be fp32 (T, H)")
     cache = kv_cache
     H = int(q.shape[1])
-    pps = _pps_min(n_req)
+    pps, split = _launch_shape(st, n_req)
     lib = _lib.load()
     stream = _lib.stream_ptr(q.device)
     _lib.check(lib.locks_mla_decode_splitk(
@@ -49,12 +65,12 @@ def mla_decode(st, q, kv_cache, block_table, seq_lens, n_req: int, scale: float,
         int(block_table.shape[1]), _lib.ptr(st.page_table), st.page_table.stride(0),
         int(st.max_pages), _lib.ptr(st.page_cnt), _lib.ptr(seq_lens), _lib.ptr(st.m_part),
         _lib.ptr(st.l_part), _lib.ptr(st.acc_part), int(n_req), H, st.D, st.Dr, st.page,
-        int(st.split), pps, float(scale), stream), "mla_decode_splitk")
+        split, pps, float(scale), stream), "mla_decode_splitk")
     _lib.check(lib.locks_mla_decode_merge(
         _lib.ptr(st.m_part), _lib.ptr(st.l_part), _lib.ptr(st.acc_part), _lib.ptr(st.page_cnt),
         int(st.max_pages), _lib.ptr(out), out.stride(0), out.stride(1),
         1 if out.dtype == torch.float32 else 0, _lib.ptr(lse) if lse is not None else None,
-        lse.stride(0) if lse is not None else 0, int(n_req), H, st.D, int(st.split), pps,
+        lse.stride(0) if lse is not None else 0, int(n_req), H, st.D, split, pps,
         stream), "mla_decode_merge")
 
 
