@@ -150,11 +150,15 @@ def rows_arg(st) -> int:
 
 def stream_ptr(device=None) -> int:
     """The current stream of `device` (None: of the current device) as a raw
-    pointer; torch's own raw getter, 2.1 -> 0.6 us against a Stream object."""
+    pointer; torch's own raw getter where it has one, 2.1 -> 0.6 us against a
+    Stream object."""
     import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return int(torch.cuda.current_stream(device).cuda_stream)
     if device is None:
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        return raw(torch.cuda.current_device())
     d = torch.device(device)
     if d.type != "cuda":
         raise ValueError(f"Expected a cuda device, but got: {d}")
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if d.index is None else d.index)
+    return raw(torch.cuda.current_device() if d.index is None else d.index)
