@@ -5,7 +5,7 @@ Call contract of the reference (src/locks/attention/decode.py:130-156,
 fp32 live on the state; pps = max(cdiv(page_cnt, split), pps_min) is derived
 on device; ``out`` (T, H, d) rows [0, n_req) are written in place; no host
 sync, no allocation.  K comes from the resident paged cache; V through the
-V-source seam (only the resident source exists in this build).
+V-source seam: the cache's V half or the DRAM tier (``locks.tier``).
 """
 from __future__ import annotations
 
@@ -34,13 +34,13 @@ def _kv_args(kv_cache: torch.Tensor):
     """What a kernel call takes of _split_kv's views, without making them:
     (K address, V address or None, (block, token, head) element strides,
     (num_blocks, page, n_kv, d))."""
-    shape, strides = kv_cache.shape, kv_cache.stride()
-    at = 0 if shape[0] == 2 and shape[1] != 2 else 1             # the dim of the two halves
+    n0, n1, page, n_kv, d = kv_cache.shape
+    s0, s1, st, sh, _ = kv_cache.stride()
     k = kv_cache.data_ptr()
-    v = None if at == 1 and shape[1] == 1 else k + strides[at] * kv_cache.element_size()
-    n0, n1, n2, n3 = shape[:at] + shape[at + 1:]
-    sb, st, sh, _sd = strides[:at] + strides[at + 1:]
-    return k, v, (sb, st, sh), (n0, n1, n2, n3)
+    if n0 == 2 and n1 != 2:
+        return k, k + s0 * kv_cache.element_size(), (s1, st, sh), (n1, page, n_kv, d)
+    v = None if n1 == 1 else k + s1 * kv_cache.element_size()
+    return k, v, (s0, st, sh), (n0, page, n_kv, d)
 
 
 _NO_V = ("ResidentVSource requires a resident V half; this cache is K-only: decode it with the DRAM "
@@ -116,23 +116,59 @@ def ensure_stage_b_buffers(st, device, split: int) -> None:
     st.dec_counters = torch.zeros(R, n_kv, COUNTER_STRIDE, device=device, dtype=torch.int32)
 
 
+def _launch_split(stream, q, kv, block_table, seq_lens, page_table, cnt, parts, n_req: int, G: int, split: int,
+                  pps_min: int, max_cnt: int, scale: float, tier_src=None) -> None:
+    """The split kernel from addresses and strides alone.  kv: (K address, V
+    address, K strides, V strides, (num_blocks, page, n_kv, d)); cnt: (page_cnt
+    address, request stride); parts: the addresses of m, l and acc; tier_src:
+    the DRAM tier's source select, or None."""
+    kp, vp, ks, vs, (NB, page, n_kv, d) = kv
+    q_sr, q_sh = q.stride()[:2]
+    pt_sr, pt_sh, _ = page_table.stride()
+    lib = _lib.load()
+    fn, tail = (lib.locks_decode_splitk, (stream,)) if tier_src is None else \
+        (lib.locks_decode_splitk_tier, (ctypes.addressof(tier_src), stream))
+    _lib.check(fn(
+        q.data_ptr(), q_sr, q_sh, kp, *ks, vp, *vs, NB, block_table.data_ptr(), block_table.stride(0),
+        block_table.shape[1], page_table.data_ptr(), pt_sr, pt_sh, page_table.shape[2], *cnt, seq_lens.data_ptr(),
+        *parts, n_req, n_kv, G, d, page, split, pps_min, max_cnt, scale, *tail), "decode_splitk")
+
+
+def _launch_merge(stream, parts, cnt, pt_cols: int, out, n_req: int, n_kv: int, G: int, d: int, split: int,
+                  pps_min: int, max_cnt: int) -> None:
+    """The merge of _launch_split's partials."""
+    o_sr, o_sh, _ = out.stride()
+    _lib.check(_lib.load().locks_decode_merge(
+        *parts, *cnt, pt_cols, out.data_ptr(), o_sr, o_sh, 1 if out.dtype == torch.float32 else 0, n_req, n_kv, G, d,
+        split, pps_min, max_cnt, stream), "decode_merge")
+
+
+def _view_args(k, v):
+    """_launch_split's kv of explicit (num_blocks, page, n_kv, d) views."""
+    return k.data_ptr(), v.data_ptr(), k.stride()[:3], v.stride()[:3], tuple(k.shape)
+
+
+def _ptrs(*tensors):
+    return tuple(t.data_ptr() for t in tensors)
+
+
+def _check_tier(ts, dims) -> None:
+    NB, page, n_kv, d = dims
+    if (ts.n_kv, ts.page, ts.head_dim, ts.num_blocks) != (n_kv, page, d, NB) \
+            or not 0 <= ts.layer < ts.num_layers:
+        raise ValueError(f"tier laid out for n_kv {ts.n_kv} / page {ts.page} / head_dim {ts.head_dim} / "
+                         f"{ts.num_blocks} blocks, layer {ts.layer} of {ts.num_layers}; the cache is "
+                         f"n_kv {n_kv} / page {page} / head_dim {d} / {NB} blocks")
+
+
 def decode_splitk(q, k, v, block_table, seq_lens, page_table, page_cnt, m_part, l_part,
                   acc_part, *, n_req: int, G: int, split: int, pps_min: int,
                   scale: float, max_cnt: int = 0) -> None:
     """Launch the split kernel on explicit tensors.  k, v: (NB, page, n_kv, d)
     views; page_table (R, n_kv, MP) i32; page_cnt (R, n_kv) i32."""
-    NB, page, n_kv, d = k.shape
-    lib = _lib.load()
-    _lib.check(lib.locks_decode_splitk(
-        _lib.ptr(q), q.stride(0), q.stride(1),
-        _lib.ptr(k), k.stride(0), k.stride(1), k.stride(2),
-        _lib.ptr(v), v.stride(0), v.stride(1), v.stride(2), int(NB),
-        _lib.ptr(block_table), block_table.stride(0), int(block_table.shape[1]),
-        _lib.ptr(page_table), page_table.stride(0), page_table.stride(1),
-        int(page_table.shape[2]), _lib.ptr(page_cnt), page_cnt.stride(0), _lib.ptr(seq_lens),
-        _lib.ptr(m_part), _lib.ptr(l_part), _lib.ptr(acc_part), int(n_req), int(n_kv), int(G),
-        int(d), int(page), int(split), int(pps_min), int(max_cnt), float(scale),
-        _lib.stream_ptr(q.device)), "decode_splitk")
+    _launch_split(_lib.stream_ptr(q.device), q, _view_args(k, v), block_table, seq_lens, page_table,
+                  (page_cnt.data_ptr(), page_cnt.stride(0)), _ptrs(m_part, l_part, acc_part), int(n_req), int(G),
+                  int(split), int(pps_min), int(max_cnt), float(scale))
 
 
 def decode_splitk_tier(q, k, v, block_table, seq_lens, page_table, page_cnt, m_part, l_part,
@@ -142,24 +178,10 @@ def decode_splitk_tier(q, k, v, block_table, seq_lens, page_table, page_cnt, m_p
     (``locks.tier.TierVSource.tier_src()``; attention/decode_cuda.py:178-222).
     k, v: (NB, page, n_kv, d) views of the paged cache; v is never read and
     may be any view of k's shape when the cache holds no V half."""
-    NB, page, n_kv, d = k.shape
-    ts = tier_src
-    if (ts.n_kv, ts.page, ts.head_dim, ts.num_blocks) != (n_kv, page, d, NB) \
-            or not 0 <= ts.layer < ts.num_layers:
-        raise ValueError(f"tier laid out for n_kv {ts.n_kv} / page {ts.page} / head_dim {ts.head_dim} / "
-                         f"{ts.num_blocks} blocks, layer {ts.layer} of {ts.num_layers}; the cache is "
-                         f"n_kv {n_kv} / page {page} / head_dim {d} / {NB} blocks")
-    lib = _lib.load()
-    _lib.check(lib.locks_decode_splitk_tier(
-        _lib.ptr(q), q.stride(0), q.stride(1),
-        _lib.ptr(k), k.stride(0), k.stride(1), k.stride(2),
-        _lib.ptr(v), v.stride(0), v.stride(1), v.stride(2), int(NB),
-        _lib.ptr(block_table), block_table.stride(0), int(block_table.shape[1]),
-        _lib.ptr(page_table), page_table.stride(0), page_table.stride(1),
-        int(page_table.shape[2]), _lib.ptr(page_cnt), page_cnt.stride(0), _lib.ptr(seq_lens),
-        _lib.ptr(m_part), _lib.ptr(l_part), _lib.ptr(acc_part), int(n_req), int(n_kv), int(G),
-        int(d), int(page), int(split), int(pps_min), int(max_cnt), float(scale),
-        ctypes.addressof(tier_src), _lib.stream_ptr(q.device)), "decode_splitk_tier")
+    _check_tier(tier_src, k.shape)
+    _launch_split(_lib.stream_ptr(q.device), q, _view_args(k, v), block_table, seq_lens, page_table,
+                  (page_cnt.data_ptr(), page_cnt.stride(0)), _ptrs(m_part, l_part, acc_part), int(n_req), int(G),
+                  int(split), int(pps_min), int(max_cnt), float(scale), tier_src)
 
 
 def _check_out(out) -> None:
@@ -222,14 +244,9 @@ def decode_merge(m_part, l_part, acc_part, page_cnt, out, *, n_req: int, n_kv: i
     """LSE merge of the split partials into ``out``; ``pt_cols`` is the page
     table width the split kernel was given (page_cnt is clamped to it)."""
     _check_out(out)
-    lib = _lib.load()
-    _lib.check(lib.locks_decode_merge(
-        _lib.ptr(m_part), _lib.ptr(l_part), _lib.ptr(acc_part), _lib.ptr(page_cnt),
-        page_cnt.stride(0), int(pt_cols), _lib.ptr(out), out.stride(0), out.stride(1),
-        1 if out.dtype == torch.float32 else 0, int(n_req), int(n_kv), int(G),
-        int(acc_part.shape[-1]), int(split), int(pps_min), int(max_cnt),
-        _lib.stream_ptr(out.device)),
-        "decode_merge")
+    _launch_merge(_lib.stream_ptr(out.device), _ptrs(m_part, l_part, acc_part),
+                  (page_cnt.data_ptr(), page_cnt.stride(0)), int(pt_cols), out, int(n_req), int(n_kv), int(G),
+                  acc_part.shape[-1], int(split), int(pps_min), int(max_cnt))
 
 
 def decode_dense(q, k, v, block_table, seq_lens, m_part, l_part, acc_part, out, *, n_req: int,
@@ -261,59 +278,39 @@ def sparse_paged_decode_batched(q, kv_cache, block_table, seq_lens, st, out,
     n_req = seq_lens.shape[0]
     pps = _pps_min(n_req, st.n_kv)
     mc = page_cnt_bound(st)
-    if vsource is None and not FUSED_MERGE:
-        # the resident step's two launches, from addresses and strides alone
-        # (views and per-stage argument lists: 24 -> 13.5 us of host time a layer)
-        _check_out(out)
-        kp, vp, ks, (NB, page, n_kv, d) = _kv_args(kv_cache)
-        if vp is None:
-            raise ValueError(_NO_V)
-        lib, stream = _lib.load(), _lib.stream_ptr(q.device)
-        pt, cnt = st.page_table, st.page_cnt
-        pt_sr, pt_sh, _ = pt.stride()
-        q_sr, q_sh = q.stride()[:2]
-        o_sr, o_sh = out.stride()[:2]
-        parts = (st.m_part.data_ptr(), st.l_part.data_ptr(), st.acc_part.data_ptr())
-        cnt_p, cnt_s, cols, G, split = cnt.data_ptr(), cnt.stride(0), pt.shape[2], int(st.G), int(st.split)
-        _lib.check(lib.locks_decode_splitk(
-            q.data_ptr(), q_sr, q_sh, kp, *ks, vp, *ks, NB,
-            block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
-            pt.data_ptr(), pt_sr, pt_sh, cols, cnt_p, cnt_s, seq_lens.data_ptr(),
-            *parts, int(n_req), n_kv, G, d, page, split, pps, mc, float(scale), stream), "decode_splitk")
-        _lib.check(lib.locks_decode_merge(
-            *parts, cnt_p, cnt_s, cols, out.data_ptr(), o_sr, o_sh,
-            1 if out.dtype == torch.float32 else 0, int(n_req), int(st.n_kv), G, st.acc_part.shape[-1], split, pps, mc,
-            stream), "decode_merge")
-        return
-    k, _ = _split_kv(kv_cache)
-    if vsource is None:
-        vsource = ResidentVSource(kv_cache)
-    if vsource.SRC_ID == 1:
-        # DRAM tier (decode_cuda.py:1301-1314): split kernel with the tier's
-        # source select, then the same merge
-        _, v_res = _split_kv(kv_cache)
-        decode_splitk_tier(q, k, v_res if v_res is not None else k, block_table, seq_lens,
-                           st.page_table, st.page_cnt, st.m_part, st.l_part, st.acc_part,
-                           vsource.tier_src(), n_req=n_req, G=st.G, split=st.split,
-                           pps_min=pps, scale=scale, max_cnt=mc)
-        decode_merge(st.m_part, st.l_part, st.acc_part, st.page_cnt, out, n_req=n_req,
-                     n_kv=st.n_kv, G=st.G, split=st.split, pps_min=pps,
-                     pt_cols=st.page_table.shape[2], max_cnt=mc)
-        return
-    if vsource.SRC_ID != 0:
-        raise NotImplementedError(f"V source {vsource.SRC_ID} is not built (0 = resident, 1 = DRAM tier)")
-    v = vsource.args()[0]
-    if FUSED_MERGE:
+    source = 0 if vsource is None else vsource.SRC_ID
+    if source not in (0, 1):
+        raise NotImplementedError(f"V source {source} is not built (0 = resident, 1 = DRAM tier)")
+    if FUSED_MERGE and source == 0:
+        k, _ = _split_kv(kv_cache)
+        v = (ResidentVSource(kv_cache) if vsource is None else vsource).args()[0]
         decode_fused(q, k, v, block_table, seq_lens, st.page_table, st.page_cnt, st.m_part,
                      st.l_part, st.acc_part, st.dec_counters, out, n_req=n_req, G=st.G,
                      split=st.split, pps_min=pps, scale=scale, max_cnt=mc)
         return
-    decode_splitk(q, k, v, block_table, seq_lens, st.page_table, st.page_cnt, st.m_part,
-                  st.l_part, st.acc_part, n_req=n_req, G=st.G, split=st.split,
-                  pps_min=pps, scale=scale, max_cnt=mc)
-    decode_merge(st.m_part, st.l_part, st.acc_part, st.page_cnt, out, n_req=n_req,
-                 n_kv=st.n_kv, G=st.G, split=st.split, pps_min=pps,
-                 pt_cols=st.page_table.shape[2], max_cnt=mc)
+    # two launches, from addresses and strides alone (with views and per-stage
+    # argument lists 24 -> 13.5 us of host time a layer)
+    _check_out(out)
+    kp, vp, ks, dims = _kv_args(kv_cache)
+    vs, tier_src = ks, None
+    if source == 1:
+        # DRAM tier (decode_cuda.py:1301-1314): the tier's source select; V is
+        # not read from the cache
+        tier_src = vsource.tier_src()
+        _check_tier(tier_src, dims)
+        vp = kp if vp is None else vp
+    elif vsource is not None:
+        v = vsource.args()[0]
+        vp, vs = v.data_ptr(), v.stride()[:3]
+    elif vp is None:
+        raise ValueError(_NO_V)
+    stream, pt, G, split = _lib.stream_ptr(q.device), st.page_table, int(st.G), int(st.split)
+    cnt = (st.page_cnt.data_ptr(), st.page_cnt.stride(0))
+    acc = st.acc_part
+    parts = (st.m_part.data_ptr(), st.l_part.data_ptr(), acc.data_ptr())
+    _launch_split(stream, q, (kp, vp, ks, vs, dims), block_table, seq_lens, pt, cnt, parts, n_req, G, split, pps, mc,
+                  float(scale), tier_src)
+    _launch_merge(stream, parts, cnt, pt.shape[2], out, n_req, int(st.n_kv), G, acc.shape[-1], split, pps, mc)
 
 
 def page_cnt_bound(st) -> int:
