@@ -11,7 +11,7 @@
 //   ms = max(|mu| / 127, 1e-8); muq = clamp(rint(mu / ms), +-127)
 //   scales stored bf16 (RNE); tag = K[15, kh, 0:8].
 //
-// MI355X mapping: a wave builds 64 / page pages at once, a page on `page`
+// MI355X mapping: a wave builds up to 64 / page pages at once, a page on `page`
 // lanes, with the gram and the eigenvectors in registers (rki4_build_kernel).
 // The gram runs on v_mfma_f32_16x16x4_f32 (A and B operands are the same lane
 // values because Gm = dc dc^T); the eigendecomposition is a parallel cyclic
@@ -45,99 +45,6 @@ __host__ __device__ __forceinline__ int pages_per_wave(long items, long waves, i
     int g = 1;
     for (int k = 1; k < gw; ++k) g += items > k * n ? 1 : 0;
     return g;
-}
-
-// Per-wave LDS image of one page of locks_pack_rki4: PG tokens x D dims and
-// the caller's eigenvectors.
-template <int D, int PG>
-struct WaveLds {
-    float dc[PG][D + 1];         // centred page (padded rows)
-    float mu[D];
-    float U[PG][PG + 1];         // eigenvectors (columns)
-    float S8[BD_RNK];
-    int col[BD_RNK];             // eigen column of basis r (ascending top-8)
-};
-
-// quantize + pack one page from mu (LDS), dc (LDS), U8 = U[:, col[r]],
-// S8 (LDS), writing the six slab rows.  Lane l owns the packed bytes
-// j = l + 64 k (d = 2j, 2j + 1).
-template <int D, int PG>
-__device__ __forceinline__ void pack_page(WaveLds<D, PG>& L, long row, const SlabRows& S) {
-    constexpr int NK = (D / 2 + 63) / 64;      // packed bytes per lane (d = 64: lanes < 32)
-    const int lane = threadIdx.x & 63;
-    auto own = [&](int k) { return lane + 64 * k < D / 2; };
-    // V[d][r]: sequential over t, separately rounded
-    float V[NK][2][BD_RNK];
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int d = 2 * (lane + 64 * k) + e;
-#pragma unroll
-            for (int r = 0; r < BD_RNK; ++r) {
-                // a compiler barrier keeps one column's operands live at a
-                // time (hoisting all 16 x 8 basis values costs ~130 VGPRs and
-                // halves the occupancy)
-                asm volatile("" ::: "memory");
-                float acc = 0.f;
-                const int c = L.col[r];
-                if (own(k))
-                    for (int t = 0; t < PG; ++t) acc = __fadd_rn(acc, __fmul_rn(L.dc[t][d], L.U[t][c]));
-                V[k][e][r] = __fdiv_rn(acc, L.S8[r]);
-            }
-        }
-    // per-column absmax over d
-    float vsc[BD_RNK];
-#pragma unroll
-    for (int r = 0; r < BD_RNK; ++r) {
-        float am = 0.f;
-#pragma unroll
-        for (int k = 0; k < NK; ++k) am = fmaxf(am, fmaxf(fabsf(V[k][0][r]), fabsf(V[k][1][r])));
-        am = wave_max(am);
-        vsc[r] = fmaxf(__fdiv_rn(am, 7.f), 1e-8f);
-    }
-    uint8_t* vrow = S.v4 + row * S.sv4;
-#pragma unroll
-    for (int r = 0; r < BD_RNK; ++r)
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-            const int lo = (int)fminf(fmaxf(rintf(__fdiv_rn(V[k][0][r], vsc[r])), -8.f), 7.f);
-            const int hi = (int)fminf(fmaxf(rintf(__fdiv_rn(V[k][1][r], vsc[r])), -8.f), 7.f);
-            if (own(k)) vrow[r * (D / 2) + lane + 64 * k] = (uint8_t)((lo & 15) | ((hi & 15) << 4));
-        }
-    if (lane < BD_RNK) reinterpret_cast<uint16_t*>(S.vs + row * S.svs)[lane] = f32_to_bf16(vsc[lane]);
-    // coefficients: lane t < PG owns token t
-    if (lane < PG) {
-        const int t = lane;
-        float C[BD_RNK];
-        float am = 0.f;
-#pragma unroll
-        for (int r = 0; r < BD_RNK; ++r) {
-            C[r] = __fmul_rn(L.U[t][L.col[r]], L.S8[r]);
-            am = fmaxf(am, fabsf(C[r]));
-        }
-        const float csc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f);
-        int8_t* crow = reinterpret_cast<int8_t*>(S.c8 + row * S.sc8) + t * BD_RNK;
-#pragma unroll
-        for (int r = 0; r < BD_RNK; ++r)
-            crow[r] = (int8_t)fminf(fmaxf(rintf(__fdiv_rn(C[r], csc)), -127.f), 127.f);
-        reinterpret_cast<uint16_t*>(S.cs + row * S.scs)[t] = f32_to_bf16(csc);
-    }
-    // centroid
-    float am = 0.f;
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-        if (own(k)) am = fmaxf(am, fmaxf(fabsf(L.mu[2 * (lane + 64 * k)]), fabsf(L.mu[2 * (lane + 64 * k) + 1])));
-    am = wave_max(am);
-    const float msc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f);
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int d = 2 * (lane + 64 * k) + e;
-            if (own(k)) reinterpret_cast<int8_t*>(S.mu + row * S.smu)[d] = (int8_t)fminf(fmaxf(rintf(__fdiv_rn(L.mu[d], msc)), -127.f), 127.f);
-        }
-    if (lane == 0) *reinterpret_cast<uint16_t*>(S.mus + row * S.smus) = f32_to_bf16(msc);
 }
 
 __device__ __forceinline__ long readlane64(long v, int l) {
@@ -192,13 +99,15 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // is register arithmetic and only the gram's column half moves data between
 // lanes (PG ds_bpermute per step, no LDS storage).  With one page per wave and
 // both matrices in LDS the build was bound by its LDS accesses (page 16: ~47
-// per step and page) and, one page alone, by their latency.  Same roundings in
-// the same order, so the records keep their bytes.  Measured, before -> after:
-//   8 layers x 2048 pages x 8 heads, d 128 page 16   4.06 -> 0.91 ms (7.0 ns a page)
+// per step and page) and, one page alone, by their latency.  The rotations round
+// as they did; the stop test sums in another order, so a page right at its bound
+// may take a sweep more or less (none of the pages compared did: bytes equal).
+// Measured, before -> after:
+//   8 layers x 2048 pages x 8 heads, d 128 page 16   4.06 -> 0.92 ms (7.0 ns a page)
 //   8 layers x 2048 latent pages, d 512              1.20 -> 0.26 ms
 //   4 layers x 512 pages x 8 heads, d 128 page 32    6.52 -> 0.96 ms
 //   4 layers x 256 pages x 8 heads, d 128 page 64    135 -> 3.85 ms
-//   32 layers x 8 heads x 4 pages (one a wave)       82 -> 60 us
+//   32 layers x 8 heads x 4 pages (one a wave)       82 -> 58 us
 // What bounds page 16 now: the Jacobi takes 2/3 of the time, ~120 clocks per CU
 // for a wave's step of ~140-167 VALU instructions and 23 LDS operations (18
 // exchanges), four waves a SIMD.  Both pipes are near full: the schedule from a
@@ -619,27 +528,86 @@ __global__ __launch_bounds__(256, PG == 16 && D <= 128 ? 4 : 2) void rki4_build_
     }
 }
 
-// locks_pack_rki4: quantize + pack given the caller's eigen decomposition.
+// ---- locks_pack_rki4 ----------------------------------------------------------
+// One page of PK_PG tokens x PK_D dims and the caller's eigenvectors, per wave.
+constexpr int PK_D = 128, PK_PG = 16;
+struct PackLds {
+    float dc[PK_PG][PK_D + 1];   // centred page (padded rows)
+    float mu[PK_D];
+    float U[PK_PG][PK_PG + 1];   // eigenvectors (columns, ascending: the last 8 are kept)
+    float S8[BD_RNK];
+};
+
+// quantize + pack one page, writing the six slab rows.  Lane l owns packed
+// byte l of each column (d = 2 l, 2 l + 1).
+__device__ __forceinline__ void pack_page(PackLds& L, long row, const SlabRows& S) {
+    static_assert(PK_D == 2 * kWave, "two dims per lane");
+    const int lane = threadIdx.x & 63;
+    // V[d][r]: sequential over t, separately rounded
+    float V[2][BD_RNK];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int r = 0; r < BD_RNK; ++r) {
+            // a compiler barrier keeps one column's operands live at a time
+            // (hoisting all 16 x 8 basis values costs ~130 VGPRs and halves the
+            // occupancy)
+            asm volatile("" ::: "memory");
+            float acc = 0.f;
+            for (int t = 0; t < PK_PG; ++t)
+                acc = __fadd_rn(acc, __fmul_rn(L.dc[t][2 * lane + e], L.U[t][PK_PG - BD_RNK + r]));
+            V[e][r] = __fdiv_rn(acc, L.S8[r]);
+        }
+    uint8_t* vrow = S.v4 + row * S.sv4;
+#pragma unroll
+    for (int r = 0; r < BD_RNK; ++r) {                        // per-column absmax over d
+        const float vsc = fmaxf(__fdiv_rn(wave_max(fmaxf(fabsf(V[0][r]), fabsf(V[1][r]))), 7.f), 1e-8f);
+        const int lo = (int)fminf(fmaxf(rintf(__fdiv_rn(V[0][r], vsc)), -8.f), 7.f);
+        const int hi = (int)fminf(fmaxf(rintf(__fdiv_rn(V[1][r], vsc)), -8.f), 7.f);
+        vrow[r * (PK_D / 2) + lane] = (uint8_t)((lo & 15) | ((hi & 15) << 4));
+        if (lane == r) reinterpret_cast<uint16_t*>(S.vs + row * S.svs)[r] = f32_to_bf16(vsc);
+    }
+    // coefficients: lane t < PK_PG owns token t
+    if (lane < PK_PG) {
+        const int t = lane;
+        float C[BD_RNK];
+        float am = 0.f;
+#pragma unroll
+        for (int r = 0; r < BD_RNK; ++r) {
+            C[r] = __fmul_rn(L.U[t][PK_PG - BD_RNK + r], L.S8[r]);
+            am = fmaxf(am, fabsf(C[r]));
+        }
+        const float csc = fmaxf(__fdiv_rn(am, 127.f), 1e-8f);
+        int8_t* crow = reinterpret_cast<int8_t*>(S.c8 + row * S.sc8) + t * BD_RNK;
+#pragma unroll
+        for (int r = 0; r < BD_RNK; ++r)
+            crow[r] = (int8_t)fminf(fmaxf(rintf(__fdiv_rn(C[r], csc)), -127.f), 127.f);
+        reinterpret_cast<uint16_t*>(S.cs + row * S.scs)[t] = f32_to_bf16(csc);
+    }
+    // centroid
+    const float msc = fmaxf(__fdiv_rn(wave_max(fmaxf(fabsf(L.mu[2 * lane]), fabsf(L.mu[2 * lane + 1]))), 127.f), 1e-8f);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        reinterpret_cast<int8_t*>(S.mu + row * S.smu)[2 * lane + e] =
+            (int8_t)fminf(fmaxf(rintf(__fdiv_rn(L.mu[2 * lane + e], msc)), -127.f), 127.f);
+    if (lane == 0) *reinterpret_cast<uint16_t*>(S.mus + row * S.smus) = f32_to_bf16(msc);
+}
+
 __global__ __launch_bounds__(4 * kWave) void rki4_pack_kernel(
     const float* __restrict__ mu, const float* __restrict__ dc, const float* __restrict__ S2,
     const float* __restrict__ U, const int* __restrict__ rows, int n, SlabRows S)
 {
-    constexpr int BD_D = 128, BD_PG = 16;
-    __shared__ WaveLds<BD_D, BD_PG> lds[4];
+    __shared__ PackLds lds[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    WaveLds<BD_D, BD_PG>& L = lds[wave];
+    PackLds& L = lds[wave];
     const long item = (long)blockIdx.x * 4 + wave;
     if (item >= n) return;
-    for (int i = lane; i < BD_PG * BD_D; i += kWave) L.dc[i / BD_D][i % BD_D] = dc[item * BD_PG * BD_D + i];
-    for (int i = lane; i < BD_D; i += kWave) L.mu[i] = mu[item * BD_D + i];
-    for (int i = lane; i < BD_PG * BD_PG; i += kWave) L.U[i / BD_PG][i % BD_PG] = U[item * BD_PG * BD_PG + i];
-    if (lane < BD_RNK) {
-        const int c = BD_PG - BD_RNK + lane;                 // ascending input: top 8 = last 8
-        L.col[lane] = c;
-        L.S8[lane] = __fsqrt_rn(fmaxf(S2[item * BD_PG + c], 1e-10f));
-    }
+    for (int i = lane; i < PK_PG * PK_D; i += kWave) L.dc[i / PK_D][i % PK_D] = dc[item * PK_PG * PK_D + i];
+    for (int i = lane; i < PK_D; i += kWave) L.mu[i] = mu[item * PK_D + i];
+    for (int i = lane; i < PK_PG * PK_PG; i += kWave) L.U[i / PK_PG][i % PK_PG] = U[item * PK_PG * PK_PG + i];
+    if (lane < BD_RNK) L.S8[lane] = __fsqrt_rn(fmaxf(S2[item * PK_PG + PK_PG - BD_RNK + lane], 1e-10f));
     wave_lds_sync();
-    pack_page<BD_D, BD_PG>(L, rows[item], S);
+    pack_page(L, rows[item], S);
 }
 
 // ---- refresh lifecycle: which blocks to (re)build --------------------------
@@ -824,7 +792,7 @@ extern "C" int32_t locks_pack_rki4(const float* mu, const float* dc, const float
                                    int8_t* c8, uint16_t* cs, int8_t* mu8, uint16_t* mus,
                                    const int64_t* slab_row_bytes, void* stream)
 {
-    LOCKS_REQUIRE(head_dim == 128 && page == 16,
+    LOCKS_REQUIRE(head_dim == PK_D && page == PK_PG,
                   "locks_pack_rki4: geometry d=%d page=%d unsupported (this entry: 128/16)", head_dim, page);
     LOCKS_REQUIRE(n >= 0, "locks_pack_rki4: n=%d < 0", n);
     LOCKS_REQUIRE(mu && dc && S2 && U && rows && v4 && vs && c8 && cs && mu8 && mus,

@@ -141,11 +141,11 @@ __device__ uint32_t block_kth_largest(const uint32_t* keys, int n, int k, int* h
 
 // Ordered emission of the top-k of keys[0, n) (page order) under
 // (key descending, index ascending): every key > tau plus the first
-// (k - #(>tau)) keys == tau.  Writes out_page[pos] = page_of(i) and, if
-// out_key != nullptr, out_key[pos] = key.  Returns the count (== k).
+// (k - #(>tau)) keys == tau.  Writes out_page[pos] = page_of(i); returns the
+// count (== k).
 template <int BLK, class PageOf>
 __device__ int emit_topk(const uint32_t* keys, int n, int k, uint32_t tau, PageOf page_of,
-                         int* out_page, uint32_t* out_key, int* wsum) {
+                         int* out_page, int* wsum) {
     const int tid = threadIdx.x;
     const int E = cdiv(n, BLK);
     const int i0 = min(tid * E, n), i1 = min(i0 + E, n);
@@ -181,11 +181,7 @@ __device__ int emit_topk(const uint32_t* keys, int n, int k, uint32_t tau, PageO
             const bool in = b0 + j < i1;
             bool kp = in && u[j] > tau;
             if (in && u[j] == tau) { kp = er < quota; ++er; }
-            if (kp) {
-                out_page[pos] = pg[j];
-                if (out_key) out_key[pos] = u[j];
-                ++pos;
-            }
+            if (kp) out_page[pos++] = pg[j];
         }
     }
     return total;
@@ -260,7 +256,7 @@ __device__ void finish_row(long rk, int n_pages, int n_sel_hi, int n_sink, int b
     __syncthreads();                    // the candidates are in global memory
     const uint32_t tau = block_kth_largest<BLK>(kk, N, b, hist, s3);
     const int nsel_w = emit_topk<BLK>(kk, N, b, tau, [&](int i) { return pp[i]; },
-                                      trow + n_sink, nullptr, wsum);
+                                      trow + n_sink, wsum);
     const int cnt = n_sink + nsel_w + (n_pages - n_sel_hi);
     for (int i = tid; i < n_sink; i += BLK) trow[i] = i;
     for (int i = n_sink + nsel_w + tid; i < cnt; i += BLK) trow[i] = n_sel_hi + (i - n_sink - nsel_w);

@@ -169,13 +169,13 @@ def _random_select_inputs(seed, n_kv, G, seq_lens, MP, st, ties=None):
 
 @pytest.mark.parametrize("combine", ["max", "nrm"])
 @pytest.mark.parametrize("seq_lens,n_kv,G,bp", [
-    ([16384], 8, 4, 126),            # one chunk (fused finish)
+    ([16384], 8, 4, 126),            # whole-row kernel, 4 pages/thread
     ([131072], 8, 4, 126),           # Llama 128K: whole-row kernel, 8 pages/thread
-    ([200000], 2, 16, 126),          # whole-row kernel, 16 pages/thread, G=16
+    ([200000], 2, 16, 126),          # chunks of 1024 pages, G=16
     ([40000], 2, 4, 1000),           # whole-row kernel, 4 pages/thread, large b
     ([1 << 20], 2, 16, 126),         # 1M context, 32 chunks
     ([262144, 196608, 131072, 65536], 2, 16, 126),   # ragged batch
-    ([100000], 2, 4, 5000),          # large b (spills past the LDS cap)
+    ([100000], 2, 4, 5000),          # whole-row kernel, 8 pages/thread, large b
     ([400000], 2, 4, 5000),          # histogram (band) route: b * chunks > register finisher
     ([1 << 20], 2, 16, 6553),        # 1M at the default 10 % budget: band route
     ([262144], 2, 16, 1638),         # 16 candidates per thread in the finisher
