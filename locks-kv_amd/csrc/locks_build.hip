@@ -550,22 +550,25 @@ __device__ __forceinline__ void pack_page(PackLds& L, long row, const SlabRows& 
 #pragma unroll
         for (int r = 0; r < BD_RNK; ++r) {
             // a compiler barrier keeps one column's operands live at a time
-            // (hoisting all 16 x 8 basis values costs ~130 VGPRs and halves the
-            // occupancy)
             asm volatile("" ::: "memory");
             float acc = 0.f;
             for (int t = 0; t < PK_PG; ++t)
                 acc = __fadd_rn(acc, __fmul_rn(L.dc[t][2 * lane + e], L.U[t][PK_PG - BD_RNK + r]));
             V[e][r] = __fdiv_rn(acc, L.S8[r]);
         }
+    // per-column absmax over d (all of them before the first code: taken column by
+    // column, the loads of every column move up and hold 480 VGPRs against 74)
+    float vsc[BD_RNK];
+#pragma unroll
+    for (int r = 0; r < BD_RNK; ++r)
+        vsc[r] = fmaxf(__fdiv_rn(wave_max(fmaxf(fabsf(V[0][r]), fabsf(V[1][r]))), 7.f), 1e-8f);
     uint8_t* vrow = S.v4 + row * S.sv4;
 #pragma unroll
-    for (int r = 0; r < BD_RNK; ++r) {                        // per-column absmax over d
-        const float vsc = fmaxf(__fdiv_rn(wave_max(fmaxf(fabsf(V[0][r]), fabsf(V[1][r]))), 7.f), 1e-8f);
-        const int lo = (int)fminf(fmaxf(rintf(__fdiv_rn(V[0][r], vsc)), -8.f), 7.f);
-        const int hi = (int)fminf(fmaxf(rintf(__fdiv_rn(V[1][r], vsc)), -8.f), 7.f);
+    for (int r = 0; r < BD_RNK; ++r) {
+        const int lo = (int)fminf(fmaxf(rintf(__fdiv_rn(V[0][r], vsc[r])), -8.f), 7.f);
+        const int hi = (int)fminf(fmaxf(rintf(__fdiv_rn(V[1][r], vsc[r])), -8.f), 7.f);
         vrow[r * (PK_D / 2) + lane] = (uint8_t)((lo & 15) | ((hi & 15) << 4));
-        if (lane == r) reinterpret_cast<uint16_t*>(S.vs + row * S.svs)[r] = f32_to_bf16(vsc);
+        if (lane == r) reinterpret_cast<uint16_t*>(S.vs + row * S.svs)[r] = f32_to_bf16(vsc[r]);
     }
     // coefficients: lane t < PK_PG owns token t
     if (lane < PK_PG) {
